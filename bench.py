@@ -31,12 +31,12 @@ METRIC = "INT8 train tokens/s (12L, 2048 tok); block-32 GEMM TOPS & % i8 MFMA pe
 PEAK_I8 = 5.0e15          # MI355X dense int8 MFMA, ops/s
 PEAK_HBM = 8.0e12         # bytes/s
 # The format's bound: every output needs, per K-block, the exact rounding of that block's product. k_gemm spends
-# 4 VALU lane-operations per output and K-block on it (fp64 cvt, ldexp by the row shift, fma by the column scale
-# plus the rounding constant, int add), and MI355X issues 64 VALU lane-ops per clock per CU (4 SIMD16, wave64)
-# on 256 CUs at 2.4 GHz. A GEMM of 2 M N K ops can therefore not beat 2 BLK / 4 x 39.3e12 ops/s however the MFMA
-# is fed: 629 TOP/s at BLK = 32, 12.6% of the i8 MFMA peak.
+# 3 VALU lane-operations per output and K-block on it at BLK = 32 (two fp32 FMAs, half a three-operand add, half a
+# three-operand or that watches the range), and MI355X issues 64 VALU lane-ops per clock per CU (4 SIMD16, wave64)
+# on 256 CUs at 2.4 GHz. A GEMM of 2 M N K ops can therefore not beat 2 BLK / 3 x 39.3e12 ops/s however the MFMA
+# is fed: 839 TOP/s at BLK = 32, 16.8% of the i8 MFMA peak. (At BLK = 128 the rounding takes 4.)
 VALU_LANE_OPS = 256 * 64 * 2.4e9
-VALU_POR_BLOCO = 4.0
+VALU_POR_BLOCO = {32: 3.0, 128: 4.0}
 
 CONFIGS = {
     "b4": dict(V=256, D=512, H=8, FF=2048, L=12, T=256, Bt=8, BLK=32, r16=False,
@@ -213,13 +213,14 @@ def mede_dw_lote(O, ops, c, rep=7):
     del grafo
     ms = sorted(vezes)[len(vezes) // 2]
     ops_alg = sum(2 * M * N * K for _, M, N in formas)
-    tiles = sum((M // 32) * (N // 128) for _, M, N in formas)
+    r = 2 if all(M % 64 == 0 for _, M, _ in formas) and sum((M // 64) * (N // 128) for _, M, N in formas) >= (512 if blk == 32 else 256) else 1
+    tiles = sum((M // (32 * r)) * (N // 128) for _, M, N in formas)
     lote = 64                                   # GEMMs per grouped launch (LOTE_G)
     nk = 1
-    while nk < 4 and tiles * 2 * nk <= 1024 and (K // blk) >= 8 * nk:
+    while nk < 4 // r and tiles * r * 2 * nk <= 1024 and (K // blk) >= 8 * nk:
         nk *= 2
     return dict(ms=ms, ms_each=[round(x, 4) for x in vezes], ops=ops_alg, gemms=len(formas), K=K, launches=(len(formas) + lote - 1) // lote,
-                symbol=f"k_gemm_lote<{blk}, {nk}, 1>", workgroups=tiles, threads=256 * nk)
+                symbol=f"k_gemm_lote<{blk}, {nk}, {r}>", workgroups=tiles, threads=256 * r * nk)
 
 
 def mede_dw_no_passo(ops, reg, c, rep=15):
@@ -322,7 +323,7 @@ def tabela_kernels(c, gem, dw, ops2, ot, ms_passo):
     roofline figure: TOP/s against the i8 MFMA peak and the format's VALU bound (GEMMs), or algorithmic GB/s
     against 8 TB/s."""
     L = c["L"]
-    lim = 2 * c["BLK"] / VALU_POR_BLOCO * VALU_LANE_OPS
+    lim = 2 * c["BLK"] / VALU_POR_BLOCO[c["BLK"]] * VALU_LANE_OPS
     lin = []
     for nome, v in gem.items():
         if nome.startswith("dW "):
@@ -787,7 +788,7 @@ def main():
     ot = mede_otimizador_e_transpostas(O, ops, c)
     ops2 = mede_ops(O, ops, c, reg)
     tabela = tabela_kernels(c, gem, dw, ops2, ot, ms_passo)
-    lim = 2 * c["BLK"] / VALU_POR_BLOCO * VALU_LANE_OPS
+    lim = 2 * c["BLK"] / VALU_POR_BLOCO[c["BLK"]] * VALU_LANE_OPS
     # the roofline line is the single kernel with the most time per step (the attention rows are four-launch
     # sequences); at configs 4 and 5 that is the grouped weight-gradient launch (k_gemm_lote), whose algorithmic
     # work is 2 M N K summed over its GEMMs
@@ -811,7 +812,7 @@ def main():
     roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": PEAK_I8 / 1e12, "unit": "TOP/s",
             "frac": achieved / PEAK_I8, "traffic": traf, "kernel": kern, "avg_ms": avg_ms, "launch_ms_samples": amostras,
             "format_bound": {"bound": "valu", "peak": lim / 1e12, "unit": "TOP/s", "frac": achieved / lim,
-                             "valu_lane_ops_per_output_block": VALU_POR_BLOCO, "valu_lane_ops_per_s": VALU_LANE_OPS}}
+                             "valu_lane_ops_per_output_block": VALU_POR_BLOCO[c["BLK"]], "valu_lane_ops_per_s": VALU_LANE_OPS}}
     res = {"metric": METRIC, "value": tps, "unit": "tokens/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
            "ms_per_step": ms_passo, "higher_is_better": True, "scaling": "weak",
            "vs_baseline": tps / c["publicado"] if c.get("publicado") else None, "dtype": "int8",

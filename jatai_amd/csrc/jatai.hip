@@ -81,8 +81,8 @@ static void lds_max(K* k, size_t lds) {
 
 #define POR_BLK(CHAMADA) (g_blk == 32 ? (CHAMADA(32)) : (CHAMADA(128)))
 
-// K-splits inside a workgroup: doubled (up to 4) while tiles x splits stays within g_alvo_wg and each split
-// keeps at least four K-blocks. A split adds a group of 4 waves to the workgroup: more resident waves per SIMD to
+// K-splits inside a workgroup: doubled (up to 4) while tiles x rows / 32 x splits stays within g_alvo_wg and each split
+// keeps at least four K-blocks. A split adds a group of 4 R waves to the workgroup: more resident waves per SIMD to
 // hide LDS and MFMA latency under the VALU rounding work, as long as the grid does not already fill the chip
 // (1024 = 256 CUs x 4 SIMDs). (Each K-split holds two stage buffers in LDS -- 10 KiB each at BLK=32, 21 KiB at
 // BLK=128, 160 KiB per workgroup.) Up to 4 splits for modes 0-2 at BLK=32 (mode 2 at 1024 threads: 60 VGPRs, no
@@ -92,14 +92,16 @@ static void lds_max(K* k, size_t lds) {
 static bool k_ok(int K) { return K <= 4096 || (K <= 65536 && (K / g_blk) % 16 == 0); }
 
 // Tile of 32 R rows. Forced by jt_gemm_bm: 64 (R = 2) or 128 (R = 4), falling back to the tallest tile that
-// divides M (every M here is a multiple of 32). Automatic: R = 1, except the fused ReLU^2 GEMMs (modes 3 and 4)
-// when 128-row tiles make one or two workgroups per CU -- measured on MI355X at M = N = 2048, K = 512 (config 4):
-// 20.4 / 19.7 us against 21.5 / 21.2 at 32 rows; with many more tiles (config 5, M = 16384) and at every other
-// step shape 32 rows are fastest.
-static int gemm_r(int M, int N = 0, int modo = 0) {
+// divides M (every M here is a multiple of 32). Automatic: 64 rows where that leaves at least TILES_64 tiles, 1.5 per CU
+// at BLK = 32 (each stage's B rows then serve twice the rows; us at 32 and 64 rows: 2048 x 1536, K = 512, 384 tiles,
+// 14.2 and 14.0; 2048 x 2048, K = 512, ReLU^2, 20.0 and 17.0; 4096 x 1024, K = 1024: 27.7 and 23.1; 16384 x 512, K = 2048:
+// 91 and 79), 1 per CU at BLK = 128 (2048 x 1024, K = 256, ReLU^2: 7.25 and 7.05; 16384 x 1024, K = 1024: 67 and 58);
+// below that 32 rows, whose K-splits fill the chip (2048 x 512, K = 2048: 16.7 in 4 splits, 64 rows in 2: 23.0). 128 rows
+// measured within 3% of 64 where they fill the chip and slower elsewhere.
+static long long tiles_64() { return g_blk == 32 ? 512 : 256; }
+static int gemm_r(int M, int N) {
     int r = g_gemm_bm >= 128 ? 4 : g_gemm_bm >= 64 ? 2 : 1;
-    const long long t128 = (long long)(M / 128) * (N / 128);
-    if (g_gemm_bm == 0 && (modo == 3 || modo == 4) && t128 >= 256 && t128 <= 512) r = 4;
+    if (g_gemm_bm == 0 && M % 64 == 0 && (long long)(M / 64) * (N / 128) >= tiles_64()) r = 2;
     while (r > 1 && M % (32 * r)) r /= 2;
     return r;
 }
@@ -107,10 +109,10 @@ static int gemm_divisoes_r(int M, int N, int K, int modo, int r) {
     const long long tiles = (long long)(M / (32 * r)) * (N / gemm::BN);
     const int nb = K / g_blk, ksmax = std::min((g_blk == 32 && modo < 3) ? 4 : 2, 4 / r);   // 256 R KS <= 1024 threads
     int ks = 1;
-    while (ks < ksmax && tiles * 2 * ks <= g_alvo_wg && nb >= 8 * ks) ks *= 2;
+    while (ks < ksmax && tiles * r * 2 * ks <= g_alvo_wg && nb >= 8 * ks) ks *= 2;
     return ks;
 }
-static int gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes_r(M, N, K, modo, gemm_r(M, N, modo)); }
+static int gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes_r(M, N, K, modo, gemm_r(M, N)); }
 
 extern "C" {
 
@@ -179,7 +181,7 @@ int jt_bloco_atual() { return g_blk; }
 // No reference counterpart: the K-split count jt_gemm_f uses for a shape (workgroup = 256 x splits threads).
 int jt_gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes(M, N, K, modo); }
 // No reference counterpart: the tile rows (32, 64 or 128) jt_gemm_f uses for a shape and mode.
-int jt_gemm_tile(int M, int N, int modo) { return 32 * gemm_r(M, N, modo); }
+int jt_gemm_tile(int M, int N, int modo) { (void)modo; return 32 * gemm_r(M, N); }
 }  // extern "C"
 // modes 0-4 (jt_gemm_f) and 6 (jt_gemm_soma16)
 static int gemm_f(const void* A, const void* EA, const void* B, const void* EB, void* Cm, void* CE, void* C32, void* Ce, const void* Xm,
@@ -187,7 +189,7 @@ static int gemm_f(const void* A, const void* EA, const void* B, const void* EB, 
     using namespace gemm;
     if (M <= 0 || N <= 0 || K <= 0 || M % BM || N % BN || K % g_blk || !k_ok(K)) return (int)hipErrorInvalidValue;
     if (!alinhados(A, EA, B, EB, Cm, CE, C32, Ce, Xm, XE, Om2, OE2)) return (int)hipErrorInvalidValue;
-    const int nb = K / g_blk, r = gemm_r(M, N, modo);
+    const int nb = K / g_blk, r = gemm_r(M, N);
     // mode 4 with Om2 (T(gh)) and mode 3 with C32, Ce (T(a)): the transposed copy needs a single K-split (BLK = 32 only)
     if (modo == 4 && (Om2 || OE2) && (g_blk != 32 || !Om2 || !OE2)) return (int)hipErrorInvalidValue;
     if (modo == 3 && (C32 || Ce) && (g_blk != 32 || !C32 || !Ce)) return (int)hipErrorInvalidValue;
@@ -252,8 +254,15 @@ int jt_gemm_lote(const void* entradas, int n, int kid) {
         L.n = std::min(LOTE_G, n - base);
         L.K = e[base].K;
         L.compacto = e[base].compacto;
-        int r = 4;                                                   // the tallest forced tile every M of the group allows
-        for (int i = 0; i < L.n; i++) r = std::min(r, gemm_r(e[base + i].M > 0 ? e[base + i].M : 32));
+        // the tallest forced tile every M of the group allows, or 64 rows by the rule of gemm_r with the group's tiles
+        int r = g_gemm_bm == 0 ? 2 : 4;
+        long long t64 = 0;
+        for (int i = 0; i < L.n; i++) {
+            const int Mi = e[base + i].M > 0 ? e[base + i].M : 32;
+            r = std::min(r, g_gemm_bm == 0 ? (Mi % 64 == 0 ? 2 : 1) : gemm_r(Mi, 0));
+            t64 += (long long)(Mi / 64) * (std::max(e[base + i].N, 0) / BN);
+        }
+        if (g_gemm_bm == 0 && t64 < tiles_64()) r = 1;
         long long tot = 0;
         for (int i = 0; i < L.n; i++) {
             const EntradaG& x = e[base + i];
@@ -270,7 +279,7 @@ int jt_gemm_lote(const void* entradas, int n, int kid) {
         // K-splits for the whole group, by the rule of jt_gemm_f with the group's tile count
         const int nb = L.K / g_blk, ksmax = std::min(g_blk == 32 ? 4 : 2, 4 / r);
         int ks = 1;
-        while (ks < ksmax && tot * 2 * ks <= g_alvo_wg && nb >= 8 * ks) ks *= 2;
+        while (ks < ksmax && tot * r * 2 * ks <= g_alvo_wg && nb >= 8 * ks) ks *= 2;
         const size_t lds = gemm_lds(nb, ks, g_blk, r, gemm::CTAB_LOTE);
 #define L_(BL, S, RR) (lds_max(k_gemm_lote<BL, S, RR>, lds), k_gemm_lote<BL, S, RR><<<(unsigned)tot, 256 * RR * S, lds, g_stream>>>(L, kid + base))
         if (r == 4) { if (g_blk == 32) L_(32, 1, 4); else L_(128, 1, 4); }

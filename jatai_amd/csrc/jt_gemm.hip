@@ -4,17 +4,29 @@
 // p_ijb = sum_{k in b} a_ik b_jk (one MFMA per 32 values of K), then acc_ij += rnd(p_ijb << 4, sa + sb) with
 // sa = RA_i - ea_ib, sb = RB_j - eb_jb, round half to even; base_ij = RA_i + RB_j - 4.
 //
-// The rounding runs in fp64 with the round-to-nearest-even of the FMA itself:
+// The rounding is the round-to-nearest-even of a floating-point sum. At BLK = 32 (|p| <= 2^19) it runs in fp32:
+//   - the MFMA accumulates onto MAGICO, the bits of 1.5 2^23, so its result's bits are the float f = 1.5 2^23 + p and
+//     the conversion costs nothing;
+//   - y = fma(f, 2^-sb, -1.5 2^23 2^-sb) = p 2^-sb, exact (the constants are one pair per column and block);
+//   - t = fma(y, 2^(4 - sa), 1.5 2^23): floats in [2^23, 2^24) are spaced by 1, so the one rounding is rnd(p << 4,
+//     sa + sb), and t's bits are MAGICO plus that integer;
+//   - two blocks' bits are added by one v_add3, and MAGICO times the number of blocks is taken off at the end.
+// The sum leaves [2^23, 2^24] only where |p| > 2^18 at sa = sb = 0; bit 23 of t's bits then says so (one v_or3 per two
+// values, tested once per stage), and the exact sum is added another way. Per output and K-block: fma, fma, half an
+// add3, half an or3 = 3 VALU operations, against 4 in fp64. This per-block VALU work, not the MFMA, bounds the kernel:
+// per wave and stage of two blocks the compiled loop has 111 VALU instructions where the fp64 form had 150. At M = 16384
+// (N x K): 1536 x 512 94 -> 74 us, 512 x 2048 with the R16 add 122 -> 84, 2048 x 512 ReLU^2 131 -> 112 and its backward
+// 131 -> 103; at M = 2048: 512 x 2048 18.2 -> 15.9, 2048 x 512 18.5 -> 14.6 (launches back to back).
+// At BLK = 128 the rounding is a quarter as frequent and runs in fp64, whose code holds fewer registers there:
 //   g = fma(ldexp(double(p), 4 - sa), 2^-sb, 1.5 * 2^52).
 // ldexp and the product by a power of two are exact, and |p * 2^(4 - sa - sb)| < 2^26 (|p| <= 128 * 128 * BLK),
 // so the exact sum lies in [2^52, 2^53), where the spacing of doubles is 1: the FMA's one rounding is
 // rnd(p << 4, sa + sb), and the low 32 bits of g are that integer in two's complement (1.5 * 2^52 has zero low
-// bits). The row term is a 32-bit ldexp operand and the column term one double per column and block, so per
-// output and K-block the work is cvt, ldexp, fma and add: 4 VALU ops, against 9 in integer form. This per-block
-// VALU work, not the MFMA, bounds the kernel.
+// bits). The row term is a 32-bit ldexp operand and the column term one double per column and block: cvt, ldexp, fma
+// and add. (In fp32 there: 14.7 us against 6.5 at 2048 x 768, K = 256 with two K-splits, from spilled stage registers.)
 //
-// Tiling: a workgroup of 4 R x KS waves owns a BM x 128 output tile, BM = 32 R rows (R = 1 by default; 2 and 4 are
-// the taller tiles jt_gemm_bm selects), one 128-column block at BLK=128, four at BLK=32. K is walked in stages of
+// Tiling: a workgroup of 4 R x KS waves owns a BM x 128 output tile, BM = 32 R rows (R = 1 or 2 by the grid, gemm_r in
+// jatai.hip; 2 and 4 where jt_gemm_bm selects them), one 128-column block at BLK=128, four at BLK=32. K is walked in stages of
 // 64 (BLK=32) or 128 (BLK=128) bytes per row: wave group g (4 R waves) takes stages s = g (mod KS) and stages each
 // one through its own double-buffered LDS tile of BM + 128 rows (BM of A, 128 of B) with coalesced loads, issued
 // two stages ahead of the MFMAs; wave w of the group computes the 32 x 32 sub-tile of rows 32 (w / 4) and columns
@@ -27,8 +39,19 @@
 #include "jt_comum.h"
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 namespace gemm {
+// 1.5 2^23 and its bits: float32 numbers in [2^23, 2^24) are spaced by 1, so the bits of 1.5 2^23 + v are MAGICO + v
+constexpr float MAGICO_F = 0x1.8p23f;
+constexpr int MAGICO = 0x4b400000;
+// a + b + c modulo 2^32 in one instruction (the compiler reassociates the sum and takes two for most of them)
+__device__ __forceinline__ int soma3(int a, int b, int c) {
+    int d;
+    asm("v_add3_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+__device__ __forceinline__ float escala(int n) { return __int_as_float((127 + n) << 23); }   // 2^n
 constexpr int BM = 32, BN = 128, PAD = 4;   // BM: rows of the default tile (R = 1); a tile has 32 R rows
 // bytes of K per row and stage: 64 at BLK=32 (two blocks; smaller buffers, more resident waves), 128 at BLK=128
 // BLK=32: 64-byte rows, unpadded, with the 8-byte chunk c of tile row r stored at chunk c ^ ((r >> 1) & 7): the
@@ -67,6 +90,10 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
                                            int ef = 0, int est = 0, int ctab = 0, int compacto = 0) {
     using gemm::BN;
     using gemm::PAD;
+    using gemm::escala;
+    using gemm::soma3;
+    using gemm::MAGICO;
+    using gemm::MAGICO_F;
     using E = gemm::Est<BLK, R>;
     constexpr int SK = E::SK, LD = E::LD, STAGE = E::STAGE, VB = E::VB;
     constexpr int BM = 32 * R;                                      // tile rows
@@ -81,8 +108,9 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // values, each with its own tables (the row maxima RA, RB are over all of K). Half-size chunks keep the tables
     // of a 32-row tile at the LDS size of K = 2048, so four workgroups stay resident per CU.
     const int NBC = gemm::bloco_tab(nb, BLK, ctab);
-    const int nbt = min(nb, NBC), nch = (nb + NBC - 1) / NBC;
-    // LDS: RA [BM], RB [BN] int32 (live to the end); shift terms na[b][i] = ea_ib + 4 - RA_i (int32) and
+    // (BLK = 32: an even number of entries; the one past an odd number of blocks scales its products by 0)
+    const int nbt = BLK == 32 ? (min(nb, NBC) + 1) & ~1 : min(nb, NBC), nch = (nb + NBC - 1) / NBC;
+    // LDS: RA [BM], RB [BN] int32 (live to the end); shift terms na[b][i] = ea_ib + 4 - RA_i (int32, as termo holds it) and
     // nb[b][j] = eb_jb - RB_j (int8) of the chunk's blocks, clamped at -100 (n = na + nb <= -22 scales |p| < 2^21
     // below 1/2, i.e. to 0, as rnd(., s >= 26) does); then the stage buffers [KS][2][STAGE], which first hold the
     // chunk's raw exponent bytes and at the end the KS accumulator tiles.
@@ -104,7 +132,7 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // Stage loads through buffer resources of the tile's A rows and B rows (bounds: the tile's own bytes, so no
     // access leaves them): the stage offset is the scalar operand, the lane offsets stay fixed, and a stage takes no
     // vector address arithmetic. The last stage may extend past K (nb not a multiple of the blocks per stage): its
-    // vectors past K re-read the row's last vector instead (those bytes land in blocks >= nb, never computed).
+    // vectors past K re-read the row's last vector instead (those bytes land in a block past nb, skipped or scaled by 0).
     const auto rsA = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)row0 * K), (short)0, BM * K, 0x00020000);
     const auto rsB = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (size_t)col0 * K), (short)0, BN * K, 0x00020000);
     int voff[NL];
@@ -173,6 +201,8 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // The staged rows are sst bytes apart: with PADT, nbc + 4 when nbc is a multiple of 16, an odd number of 4-byte words, so
     // the byte reads below (consecutive threads, consecutive rows) fall in different LDS banks; rows nbc bytes
     // apart (a multiple of 64 at K >= 2048) put a wave's reads in two banks.
+    // a row's shift term n = 4 - sa as the tables hold it: the bits of the float 2^n (BLK = 32), or n
+    auto termo = [](int n) { return BLK == 32 ? __float_as_int(escala(n)) : n; };
     auto desloca_tab = [&](int nbc, int sst) {
         const int r = tid & (BM - 1), c = tid & (BN - 1);
         const int ra4 = 4 - ra_s[r], rbn = -rb_s[c];
@@ -185,7 +215,7 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
             for (int u = 0; u < U; u++) e[u] = b0 + u * SA < nbc ? (int)ea[b0 + u * SA] : 0;
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (b0 + u * SA < nbc) na_s[(b0 + u * SA) * BM + r] = max(e[u] + ra4, -100);
+                if (b0 + u * SA < nbc) na_s[(b0 + u * SA) * BM + r] = termo(max(e[u] + ra4, -100));
         }
         for (int b0 = tid >> 7; b0 < nbc; b0 += 2 * U * SB) {       // entries b * BN + c
             int e[2 * U];
@@ -247,6 +277,10 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
             else rb_s[tid - OB] = m;
         }
         __syncthreads();
+        if (nbt > nb) {
+            if (tid < BM) na_s[nb * BM + tid] = 0;
+            if (tid < BN) nb_s[nb * BN + tid] = 0;
+        }
         desloca_tab(nb, sst1);
     };
     // one chunk whose exponent rows are whole 16-byte vectors, at most 8 per row (K <= 4096): no staging. A row is
@@ -278,7 +312,7 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
                 if (j == 0) ra_s[row] = m;
                 const int ra4 = 4 - m;
 #pragma unroll
-                for (int u = 0; u < 16; u++) na_s[(16 * j + u) * BM + row] = max((int)(int8_t)(w4[u >> 2] >> (8 * (u & 3))) + ra4, -100);
+                for (int u = 0; u < 16; u++) na_s[(16 * j + u) * BM + row] = termo(max((int)(int8_t)(w4[u >> 2] >> (8 * (u & 3))) + ra4, -100));
             } else {
                 const int c = row - BM;
                 if (j == 0) rb_s[c] = m;
@@ -322,11 +356,9 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // the buffer of stage k - 1, which every wave finished reading before the barrier that ended iteration k - 1.
     // Each block's MFMAs are followed by its rounding: the MFMA latency runs under the other resident waves' VALU
     // work, and only one block's products are live (the fp64 rounding's temporaries need the registers).
+    // products start from MAGICO at BLK = 32: their bits are then the float 1.5 2^23 + p
+    const v4i mg = BLK == 32 ? v4i{MAGICO, MAGICO, MAGICO, MAGICO} : v4i{0, 0, 0, 0};
     auto produtos = [&](const char* tile, int bl, v4i (&p)[2][2]) {
-#pragma unroll
-        for (int ti = 0; ti < 2; ti++)
-#pragma unroll
-            for (int tj = 0; tj < 2; tj++) p[ti][tj] = v4i{0, 0, 0, 0};
 #pragma unroll
         for (int k = 0; k < KST; k++) {
             const int ch = (bl * KST + k) * 4 + lg;                   // 8-byte chunk of K within the stage
@@ -339,31 +371,78 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
 #pragma unroll
             for (int ti = 0; ti < 2; ti++)
 #pragma unroll
-                for (int tj = 0; tj < 2; tj++) p[ti][tj] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa[ti], fb[tj], p[ti][tj], 0, 0, 0);
+                for (int tj = 0; tj < 2; tj++) p[ti][tj] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa[ti], fb[tj], k ? p[ti][tj] : mg, 0, 0, 0);
         }
     };
-    // rnd(p << 4, sa + sb) from the row term n = 4 - sa and the column scale c = 2^-sb (see the head of this file)
-    auto rnd_fma = [](int p, int n, double c) { return __double2loint(__builtin_fma(ldexp((double)p, n), c, 0x1.8p52)); };
-    auto escala = [](int nbv) { return __hiloint2double((1023 + nbv) << 20, 0); };
-    auto arredonda = [&](int b, const v4i (&p)[2][2]) {
-        const int bt = b - b0;                                      // block index in the chunk's tables
-        const v4i na0 = *reinterpret_cast<const v4i*>(na_s + bt * BM + wr + 4 * lg);
-        const v4i na1 = *reinterpret_cast<const v4i*>(na_s + bt * BM + wr + 16 + 4 * lg);
-        const double cb0 = escala(nb_s[bt * BN + wc + lr]), cb1 = escala(nb_s[bt * BN + wc + 16 + lr]);
+    // f(ti, tj, i) for each of a wave's 16 outputs per lane
+    auto cada = [](auto f) {
 #pragma unroll
         for (int ti = 0; ti < 2; ti++)
 #pragma unroll
             for (int tj = 0; tj < 2; tj++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[ti][tj][i] += rnd_fma(p[ti][tj][i], ti ? na1[i] : na0[i], tj ? cb1 : cb0);
+                for (int i = 0; i < 4; i++) f(ti, tj, i);
+    };
+    // BLK = 32: the bits of 1.5 2^23 + rnd(p << 4, sa + sb) in place of the product's (see the head of this file)
+    auto arredonda = [&](int b, v4i (&p)[2][2]) {
+        const int bt = b - b0;                                      // block index in the chunk's tables
+        const v4f na0 = *reinterpret_cast<const v4f*>(na_s + bt * BM + wr + 4 * lg);
+        const v4f na1 = *reinterpret_cast<const v4f*>(na_s + bt * BM + wr + 16 + 4 * lg);
+        const float cb0 = escala(nb_s[bt * BN + wc + lr]), cb1 = escala(nb_s[bt * BN + wc + 16 + lr]);
+        const float d0 = -MAGICO_F * cb0, d1 = -MAGICO_F * cb1;
+        cada([&](int ti, int tj, int i) {
+            const float y = __builtin_fmaf(__int_as_float(p[ti][tj][i]), tj ? cb1 : cb0, tj ? d1 : d0);
+            p[ti][tj][i] = __float_as_int(__builtin_fmaf(y, ti ? na1[i] : na0[i], MAGICO_F));
+        });
+    };
+    // BLK = 128: acc += rnd(p << 4, sa + sb) in fp64, from the row term n = 4 - sa and the column scale c = 2^-sb
+    auto arredonda_d = [&](int b, const v4i (&p)[2][2]) {
+        const int bt = b - b0;
+        const v4i na0 = *reinterpret_cast<const v4i*>(na_s + bt * BM + wr + 4 * lg);
+        const v4i na1 = *reinterpret_cast<const v4i*>(na_s + bt * BM + wr + 16 + 4 * lg);
+        const double cb0 = __hiloint2double((1023 + nb_s[bt * BN + wc + lr]) << 20, 0);
+        const double cb1 = __hiloint2double((1023 + nb_s[bt * BN + wc + 16 + lr]) << 20, 0);
+        cada([&](int ti, int tj, int i) {
+            acc[ti][tj][i] += __double2loint(__builtin_fma(ldexp((double)p[ti][tj][i], ti ? na1[i] : na0[i]), tj ? cb1 : cb0, 0x1.8p52));
+        });
+    };
+    int nadd = 0;                                                   // blocks added at BLK = 32, each with MAGICO on top
+    auto soma_acc = [&](int v, int ti, int tj, int i) { acc[ti][tj][i] = (int)((unsigned)acc[ti][tj][i] + (unsigned)v); };
+    // a sum that left [2^23, 2^24] (|p| > 2^18 at shift 0) is still the exact float, but its bits are not MAGICO + v
+    auto corrige = [&](const v4i (&p)[2][2]) {
+        cada([&](int ti, int tj, int i) {
+            const int t = p[ti][tj][i];
+            soma_acc((int)((unsigned)((int)(__int_as_float(t) - MAGICO_F) + MAGICO) - (unsigned)t), ti, tj, i);
+        });
     };
     auto calcula = [&](const char* tile, int st) {
-#pragma unroll
-        for (int bl = 0; bl < BPS; bl++) {
-            if (st * BPS + bl >= nb) break;
-            v4i p[2][2];
-            produtos(tile, bl, p);
-            arredonda(st * BPS + bl, p);
+        v4i p[2][2];
+        produtos(tile, 0, p);
+        if constexpr (BLK == 128) {
+            arredonda_d(st, p);
+        } else {
+            arredonda(st * 2, p);
+            int f = 0;                                              // bit 23 of a sum's bits: it left [2^23, 2^24)
+            // the second block of an odd number's last stage has scales of 0 and adds nothing; 32-row tiles, whose
+            // threads hold more stage rows, still skip it: without the branch both blocks' addresses stay live in
+            // registers and spill (M = 16384, N = 1536, K = 512 at 32 rows: 76 us with it, 99 without)
+            if (R > 1 || st * 2 + 1 < nb) {
+                v4i q[2][2];
+                produtos(tile, 1, q);
+                arredonda(st * 2 + 1, q);
+                cada([&](int ti, int tj, int i) {
+                    acc[ti][tj][i] = soma3(acc[ti][tj][i], p[ti][tj][i], q[ti][tj][i]);
+                    f |= p[ti][tj][i] | q[ti][tj][i];
+                });
+                nadd += 2;
+                if (__builtin_expect(__any(f >> 23 & 1), 0)) { corrige(p); corrige(q); }
+            } else {
+                // (the same test on the bits' difference from 2^23's: a form the compiler does not share with the case
+                // above, where sharing it costs 10 VALU instructions per stage)
+                cada([&](int ti, int tj, int i) { soma_acc(p[ti][tj][i], ti, tj, i); f |= p[ti][tj][i] ^ 0x4b000000; });
+                nadd += 1;
+                if (__builtin_expect(__any((unsigned)f >> 23), 0)) corrige(p);
+            }
         }
     };
     for (int c = 0; c < nch; c++) {
@@ -408,9 +487,13 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
                 for (int tj = 0; tj < 2; tj++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-                        fora |= (int)(acc[ti][tj][i] >= T || acc[ti][tj][i] <= -T) << (8 * ti + 4 * tj + i);
+                    {
+                        const int v = (int)((unsigned)acc[ti][tj][i] - (unsigned)nadd * (unsigned)MAGICO);
+                        fora |= (int)(v >= T || v <= -T) << (8 * ti + 4 * tj + i);
+                    }
         }
     }
+    cada([&](int ti, int tj, int i) { soma_acc((int)(-(unsigned)nadd * (unsigned)MAGICO), ti, tj, i); });
 
     // ---- output stage: KS partial tiles to LDS, summed while read back in the row-block layout. The X operand
     // of modes 2 and 4 is read here, not before the K loop, so its 16 registers do not cost a resident wave.
@@ -693,7 +776,8 @@ static inline size_t gemm_lds(int nb, int ks, int blk, int R = 1, int ctab = 0) 
     using gemm::PAD;
     const int bm = 32 * R;
     nb = std::min(nb, gemm::bloco_tab(nb, blk, ctab));              // the shift tables hold one chunk of K
-    const size_t fixo = (size_t)(bm + BN) * 4 + (size_t)nb * bm * 4 + (((size_t)nb * BN + 15) & ~(size_t)15);
+    const size_t nbt = blk == 32 ? (nb + 1) & ~1 : nb;
+    const size_t fixo = (size_t)(bm + BN) * 4 + nbt * bm * 4 + ((nbt * BN + 15) & ~(size_t)15);
     const size_t stage = (size_t)(32 * R + BN) * (blk == 32 ? gemm::Est<32>::LD : gemm::Est<128>::LD);
     size_t area = (size_t)ks * 2 * stage;
     const size_t exp_bruto = (size_t)(nb + 4) * (bm + BN + 1) + 16;   // staged rows nb + 4 bytes apart, and a junk row

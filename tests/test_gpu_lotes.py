@@ -149,3 +149,30 @@ def test_modelo_dw_em_lote():
         assert float(a.passo(tok, alvo, k_lr=f["k_lr"])) == float(b.passo(tok, alvo, k_lr=f["k_lr"]))
     est = lambda m: [R.sha(host(t)) for n in m.p for t in (*m.p[n], *m.mom[n], *m.res[n])]
     assert est(a) == est(b)
+
+
+@pytest.mark.parametrize("M,N,K,bm", [(64, 128, 32, 0), (64, 128, 96, 64), (128, 256, 160, 128), (96, 128, 2080, 0), (128, 128, 4096, 64),
+                                      (128, 128, 8192, 0), (4096, 1024, 64, 0)])
+def test_gemm_arredondamento_fp32(M, N, K, bm):
+    """The fp32 rounding of the BLK = 32 GEMM at its edges, against the oracle: blocks whose product passes 2^18 at shift
+    0 (mantissas of +-127 and -128, where the rounded sum leaves its binade), ties at every shift from 5 up, shifts past
+    the last nonzero one and zero blocks, at odd and even numbers of blocks, several chunks of K and each tile; the last
+    shape takes the 64-row tile by its grid."""
+    blk = 32
+    gpu, cpu = GPU(blk), CPU(blk)
+    for caso, (espalha, satura) in enumerate(((0, 1.0), (2, 0.9), (30, 0.5))):
+        s = lambda t: R.substream(131, f"{M} {N} {K} {caso} {t}")
+        t = []
+        for nome, L in (("A", M), ("B", N)):
+            m, E = R.bloco(s(nome), L, K, blk, espalha=espalha, e0=-8, zera=0.1 if caso else 0.0)
+            cheio = (R.uniform01(s(nome + "s"), (L, K)) < satura) & (np.repeat(E, blk, 1) != R.E_ZERO)
+            m = np.where(cheio, np.where(R.uniform01(s(nome + "p"), (L, 1)) < 0.5, 127, -128), m).astype(np.int8)
+            t.append((np.ascontiguousarray(m), E))
+        gpu.ops.lib.jt_gemm_bm(bm)
+        try:
+            out = gpu.ops.gemm(*[tuple(gpu.dev(v) for v in x) for x in t], cru=True)
+        finally:
+            gpu.ops.lib.jt_gemm_bm(0)
+        ref = cpu.ops.gemm(*[tuple(torch.from_numpy(v) for v in x) for x in t], cru=True)
+        for a, b in zip(out, ref):
+            assert np.array_equal(host(a), host(b)), f"{M}x{N}x{K} case {caso}"
