@@ -33,7 +33,7 @@ void jt_atencao_linhas(int n);         /* jatai_cuda.cu:1091: query rows per thr
                                         * up to T = 128, one row per thread beyond; same bits */
 int jt_res_estocastico(int ligado);    /* jatai_cuda.cu:1087: 1 = gemm_soma's residual add rounds stochastically (0 = off, the default) */
 
-/* ---- no reference counterpart: attention kernel family at head width 64, matrix cores (1, default) or dot2 (0) */
+/* ---- no reference counterpart: attention kernel family at head widths 64, 32, 16, matrix cores (1, default) or dot2 (0) */
 void jt_atencao_mfma(int ligado);
 
 /* ---- block size: no reference counterpart (the reference fixes 128) */
@@ -143,9 +143,9 @@ int jt_perda(const void* d_alvo, const void* soma, void* out, int M, int kid);
  * guard bits of the aligned values, from 0 to 4 (the spec's is 4, ops.py:20), else hipErrorInvalidValue. */
 int jt_atencao(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, int Bt, int T, int H, int D, int GA, int kid);
 /* no reference counterpart: jt_atencao with a caller workspace of jt_atencao_ws_bytes(Bt, T, H, D) bytes (16-byte
- * aligned); same outputs. At head width 64 on matrix cores (T <= 512) k and v are converted once per (sequence,
- * head) into the workspace and each 16-row query tile's keys are split over four waves; otherwise it runs
- * jt_atencao. */
+ * aligned); same outputs. At head widths 64, 32, 16 on matrix cores (T <= 512) k and v are converted once per (sequence,
+ * head) into the workspace and each 16-row query tile's keys are split over four waves; otherwise (head widths 32, 16:
+ * also without a large enough, aligned workspace) it runs jt_atencao. */
 long long jt_atencao_ws_bytes(int Bt, int T, int H, int D);
 int jt_atencao_ws(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, int Bt, int T, int H, int D, int GA, void* ws,
                   long long ws_bytes, int kid);
@@ -156,9 +156,9 @@ int jt_atencao_back(const void* gom, const void* goE, const void* qm, const void
 int jt_atencao_ws_q(const void* qm, const void* qE, void* Om, void* OE, void* P, int Bt, int T, int H, int D, int GA, void* ws,
                     long long ws_bytes, int kid);
 /* no reference counterpart: jt_atencao_back with a caller workspace of jt_atencao_back_ws_bytes(Bt, T, H, D) bytes
- * (16-byte aligned); same outputs. At head width 64 on matrix cores (T <= 512) dO, q, k, v are converted once per
- * (sequence, head) into the workspace and each 16-row tile's partner tiles are split over four waves; otherwise
- * it runs jt_atencao_back. */
+ * (16-byte aligned); same outputs. At head widths 64, 32, 16 on matrix cores (T <= 512) dO, q, k, v are converted once
+ * per (sequence, head) into the workspace and each 16-row tile's partner tiles are split over four waves; otherwise
+ * (head widths 32, 16: also without a large enough, aligned workspace) it runs jt_atencao_back. */
 long long jt_atencao_back_ws_bytes(int Bt, int T, int H, int D);
 int jt_atencao_back_ws(const void* gom, const void* goE, const void* qm, const void* qE, const void* P, void* Gacc, void* Ge, int Bt, int T,
                        int H, int D, int GA, int limite, void* ws, long long ws_bytes, int kid);

@@ -46,7 +46,7 @@ static int g_blk = 128;                 // block size of every tensor: 32 or 128
 static int g_alvo_wg = 1024;            // GEMM K-split target: tiles x K-splits per launch
 static int g_gemm_bm = 0;               // GEMM tile rows: 0 = automatic, or 32, 64, 128 forced (jt_gemm_bm)
 static int g_linhas = 0;                // head-width-4 attention layout (jt_atencao_linhas): 1 or 2 query rows per thread, 0 automatic
-static int g_atencao_mfma = 1;          // head width 64: matrix-core attention (1) or the dot2 kernels (0)
+static int g_atencao_mfma = 1;          // head widths 64, 32, 16: matrix-core attention (1) or the dot2 kernels (0)
 
 static int fim() { return (int)hipGetLastError(); }
 // Every kernel moves 8- or 16-byte vectors: operands must be 16-byte aligned (torch allocations are 256-byte
@@ -629,6 +629,17 @@ static bool atencao_forma(int Bt, int T, int H, int D, int GA) {
     if (D / H == 4) return T % 32 == 0 && T <= 256 && H <= 64;
     return T % 64 == 0 && T <= 512;
 }
+// head width a workspace is laid out for (one that runs without it is sized as 64's)
+static int largura_ws(int hd) { return hd == 16 || hd == 32 ? hd : 64; }
+// Head widths 32 and 16 with a usable workspace: the matrix-core kernels of head width 64, at every T. One MFMA
+// takes a whole head, so the work per score is the softmax's and the dS chain's own, where the v_dot2 kernels read
+// both operands from LDS for every pair and recompute each score three times: 144 against 1529 us forward and backward
+// at 8 x 512 tokens and 16 heads of 32, 124 against 990 with heads of 16, and at the smallest, one sequence of 64 tokens
+// and 4 heads of 32, 49 against 117 (the calls' host time)
+static bool ws_estreita(int D, int H, const void* ws, long long tem, long long pede) {
+    const int hd = D / H;
+    return (hd == 32 || hd == 16) && g_atencao_mfma && D % g_blk == 0 && g_blk % hd == 0 && ws && alinhados(ws) && tem >= pede;
+}
 int jt_atencao(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, int Bt, int T, int H, int D, int GA, int kid) {
     if (!atencao_forma(Bt, T, H, D, GA)) return (int)hipErrorInvalidValue;
     if (!alinhados(qm, qE, Oacc, Oe, P)) return (int)hipErrorInvalidValue;
@@ -667,12 +678,13 @@ int jt_atencao(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, in
     return fim();
 }
 // No reference counterpart: jt_atencao with a caller workspace of jt_atencao_ws_bytes(Bt, T, H, D) bytes
-// (16-byte aligned). Same outputs as jt_atencao. At head width 64 on matrix cores (T % 64 == 0, T <= 512) it
-// converts k and v once per (sequence, head) into the workspace and splits each 16-row query tile's keys over
-// four waves; otherwise it runs jt_atencao and leaves the workspace untouched.
+// (16-byte aligned). Same outputs as jt_atencao. At head widths 64, 32 and 16 on matrix cores (T % 64 == 0,
+// T <= 512) it converts k and v once per (sequence, head) into the workspace and splits each 16-row query tile's
+// keys over four waves; otherwise it runs jt_atencao and leaves the workspace untouched. Head widths 32 and 16 also
+// run jt_atencao when the workspace is missing, too small or misaligned (head width 64 refuses that).
 long long jt_atencao_ws_bytes(int Bt, int T, int H, int D) {
     if (Bt <= 0 || H <= 0 || T <= 0 || D % H) return 0;
-    return (long long)atw::bytes_fwd((long long)Bt * H, T);
+    return (long long)atw::bytes_fwd((long long)Bt * H, T, largura_ws(D / H));
 }
 // salvo (optional): the backward's conversions of q, k, v are written there too (atw::Salvo)
 static int atencao_ws(const void* qm, const void* qE, void* O1, void* O2, void* P, int Bt, int T, int H, int D, int GA, void* ws, long long ws_bytes,
@@ -680,21 +692,28 @@ static int atencao_ws(const void* qm, const void* qE, void* O1, void* O2, void* 
     if (!alinhados(qm, qE, O1, O2, P, ws, salvo) || !ws || ws_bytes < jt_atencao_ws_bytes(Bt, T, H, D) || 64 % g_blk && g_blk % 64)
         return (int)hipErrorInvalidValue;
     const long long BH = (long long)Bt * H;
-    const atw::Ws w = atw::parte(ws, BH, T);
-    if (salvo) k_atf_prep<true><<<(unsigned)(BH * (T / 64)), 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, atw::parte_s(salvo, BH, T),
-                                                                                  T, H, D, g_blk, GA);
-    else k_atf_prep<false><<<(unsigned)(BH * (T / 64)), 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, atw::Salvo{}, T, H, D, g_blk, GA);
-    const unsigned g = (unsigned)(BH * (T / 16));
-#define L(NTW, B) k_atf<NTW, B><<<g, 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, O1, O2, (uint8_t*)P, T, H, D, g_blk, GA, kid)
-    if (bloco) { if (T <= 256) L(4, true); else L(8, true); }
-    else { if (T <= 256) L(4, false); else L(8, false); }
+    const int hd = D / H;
+    const atw::Ws w = atw::parte(ws, BH, T, hd);
+    const unsigned gp = (unsigned)(BH * (T / 64)), g = (unsigned)(BH * (T / 16));
+#define PREP(HD) k_atf_prep<HD><<<gp, 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, atw::Salvo{}, T, H, D, g_blk, GA)
+#define L(HD, NTW, B) k_atf<HD, NTW, B><<<g, 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, O1, O2, (uint8_t*)P, T, H, D, g_blk, GA, kid)
+#define LE(HD) { PREP(HD); if (T <= 256) L(HD, 4, false); else L(HD, 8, false); }
+    if (hd == 32) { LE(32) return fim(); }
+    if (hd == 16) { LE(16) return fim(); }
+    if (salvo) k_atf_prep<64, true><<<gp, 256, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, w, atw::parte_s(salvo, BH, T), T, H, D, g_blk, GA);
+    else PREP(64);
+    if (bloco) { if (T <= 256) L(64, 4, true); else L(64, 8, true); }
+    else { if (T <= 256) L(64, 4, false); else L(64, 8, false); }
+#undef LE
 #undef L
+#undef PREP
     return fim();
 }
 int jt_atencao_ws(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, int Bt, int T, int H, int D, int GA, void* ws,
                   long long ws_bytes, int kid) {
     if (!atencao_forma(Bt, T, H, D, GA)) return (int)hipErrorInvalidValue;
-    if (D / H != 64 || !g_atencao_mfma || T > 512) return jt_atencao(qm, qE, Oacc, Oe, P, Bt, T, H, D, GA, kid);
+    if ((D / H != 64 || !g_atencao_mfma || T > 512) && !ws_estreita(D, H, ws, ws_bytes, jt_atencao_ws_bytes(Bt, T, H, D)))
+        return jt_atencao(qm, qE, Oacc, Oe, P, Bt, T, H, D, GA, kid);
     return atencao_ws(qm, qE, Oacc, Oe, P, Bt, T, H, D, GA, ws, ws_bytes, false, kid);
 }
 // No reference counterpart: jt_atencao_ws writing the output quantized to block format (Om int8 [M, D], OE int8
@@ -791,14 +810,15 @@ int jt_atencao_back(const void* gom, const void* goE, const void* qm, const void
 }
 
 // No reference counterpart: jt_atencao_back with a caller workspace of jt_atencao_back_ws_bytes(Bt, T, H, D)
-// bytes (16-byte aligned). Same outputs as jt_atencao_back. At head width 64 on matrix cores (T % 64 == 0,
-// T <= 512) it converts dO, q, k, v once per (sequence, head) into the workspace and splits each 16-row tile's
-// partner tiles over four waves (4 launches; the exact variant's per-tile max |gP| in the conversion launch at
-// T <= 256, a launch of its own past that or when the forward saved the q, k, v conversions); otherwise it runs
-// jt_atencao_back.
+// bytes (16-byte aligned). Same outputs as jt_atencao_back. At head widths 64, 32 and 16 on
+// matrix cores (T % 64 == 0, T <= 512) it converts dO, q, k, v once per (sequence, head) into the workspace and splits
+// each 16-row tile's partner tiles over four waves (4 launches; the exact variant's per-tile max |gP| in the
+// conversion launch at head width 64 and T <= 256, a launch of its own otherwise or when the forward saved the q, k,
+// v conversions); otherwise it runs jt_atencao_back, as head widths 32 and 16 do when the workspace is missing, too
+// small or misaligned.
 long long jt_atencao_back_ws_bytes(int Bt, int T, int H, int D) {
     if (Bt <= 0 || H <= 0 || T <= 0 || D % H) return 0;
-    return (long long)atw::bytes_back((long long)Bt * H, T);
+    return (long long)atw::bytes_back((long long)Bt * H, T, largura_ws(D / H));
 }
 // salvo (optional, exact variant): the conversions of q, k, v saved by jt_atencao_ws_qs for the same qkv
 static int atencao_back_ws(const void* gom, const void* goE, const void* qm, const void* qE, const void* P, void* G1, void* G2, int Bt, int T,
@@ -806,7 +826,8 @@ static int atencao_back_ws(const void* gom, const void* goE, const void* qm, con
     if (!alinhados(gom, goE, qm, qE, P, G1, G2, ws, salvo) || !ws || ws_bytes < jt_atencao_back_ws_bytes(Bt, T, H, D) || 64 % g_blk && g_blk % 64)
         return (int)hipErrorInvalidValue;
     const long long BH = (long long)Bt * H;
-    atw::WsB w = atw::parte_b(ws, BH, T);
+    const int hd = D / H;
+    atw::WsB w = atw::parte_b(ws, BH, T, hd);
     const int* smx = nullptr;
     if (salvo && !limite) {                              // q, k, v read from the saved conversions
         const atw::Salvo s = atw::parte_s(const_cast<void*>(salvo), BH, T);
@@ -817,25 +838,42 @@ static int atencao_back_ws(const void* gom, const void* goE, const void* qm, con
     const int8_t *go8 = (const int8_t*)gom, *goE8 = (const int8_t*)goE, *q8 = (const int8_t*)qm, *qE8 = (const int8_t*)qE;
     const uint8_t* P8 = (const uint8_t*)P;
     const unsigned gp = (unsigned)(BH * (T / 64)), gt = (unsigned)(BH * (T / 16));
+#define RESTO(HD, NTW, LM, B)                                                                                             \
+    {                                                                                                                     \
+        k_atb2<HD, NTW, LM><<<gt, 256, 0, g_stream>>>(w, P8, T, H, D, kid);                                               \
+        k_atbqkv<HD, NTW, LM, B><<<2 * gt, 256, 0, g_stream>>>(w, P8, (int*)G1, (int16_t*)G2, T, H, D, dsb, kid);         \
+    }
 #define FASES(NTW, LM, B)                                                                                                 \
     {                                                                                                                     \
         if (!LM && smx) k_atb_prep_s<<<gp, 256, 0, g_stream>>>(go8, goE8, w, smx, T, H, D, g_blk, GA);                     \
-        else if (!LM && T <= 256) k_atb_prep<0, true><<<2 * gp, 256, 0, g_stream>>>(go8, goE8, q8, qE8, w, T, H, D, g_blk, GA); \
-        else k_atb_prep<LM><<<gp, 256, 0, g_stream>>>(go8, goE8, q8, qE8, w, T, H, D, g_blk, GA);                         \
-        if (!LM && (smx || T > 256)) k_atb1<NTW><<<gt, 256, 0, g_stream>>>(w, T, H);                                      \
-        k_atb2<NTW, LM><<<gt, 256, 0, g_stream>>>(w, P8, T, H, D, kid);                                                    \
-        k_atbqkv<NTW, LM, B><<<2 * gt, 256, 0, g_stream>>>(w, P8, (int*)G1, (int16_t*)G2, T, H, D, dsb, kid);              \
+        else if (!LM && T <= 256) k_atb_prep<64, 0, true><<<2 * gp, 256, 0, g_stream>>>(go8, goE8, q8, qE8, w, T, H, D, g_blk, GA); \
+        else k_atb_prep<64, LM><<<gp, 256, 0, g_stream>>>(go8, goE8, q8, qE8, w, T, H, D, g_blk, GA);                     \
+        if (!LM && (smx || T > 256)) k_atb1<64, NTW><<<gt, 256, 0, g_stream>>>(w, T, H);                                  \
+        RESTO(64, NTW, LM, B)                                                                                             \
     }
+#define ESTREITA(HD, NTW, LM)                                                                                             \
+    {                                                                                                                     \
+        k_atb_prep<HD, LM><<<gp, 256, 0, g_stream>>>(go8, goE8, q8, qE8, w, T, H, D, g_blk, GA);                          \
+        if (!LM) k_atb1<HD, NTW><<<gt, 256, 0, g_stream>>>(w, T, H);                                                      \
+        RESTO(HD, NTW, LM, false)                                                                                         \
+    }
+#define E_(HD) { if (T <= 256) { if (limite) ESTREITA(HD, 4, 1) else ESTREITA(HD, 4, 0) } else { if (limite) ESTREITA(HD, 8, 1) else ESTREITA(HD, 8, 0) } }
 #define VAR(B) { if (T <= 256) { if (limite) FASES(4, 1, B) else FASES(4, 0, B) } else { if (limite) FASES(8, 1, B) else FASES(8, 0, B) } }
-    if (bloco) VAR(true) else VAR(false)
+    if (hd == 32) E_(32)
+    else if (hd == 16) E_(16)
+    else if (bloco) VAR(true) else VAR(false)
 #undef VAR
+#undef E_
+#undef ESTREITA
 #undef FASES
+#undef RESTO
     return fim();
 }
 int jt_atencao_back_ws(const void* gom, const void* goE, const void* qm, const void* qE, const void* P, void* Gacc, void* Ge, int Bt, int T,
                        int H, int D, int GA, int limite, void* ws, long long ws_bytes, int kid) {
     if (!atencao_forma(Bt, T, H, D, GA)) return (int)hipErrorInvalidValue;
-    if (D / H != 64 || !g_atencao_mfma || T > 512) return jt_atencao_back(gom, goE, qm, qE, P, Gacc, Ge, Bt, T, H, D, GA, limite, kid);
+    if ((D / H != 64 || !g_atencao_mfma || T > 512) && !ws_estreita(D, H, ws, ws_bytes, jt_atencao_back_ws_bytes(Bt, T, H, D)))
+        return jt_atencao_back(gom, goE, qm, qE, P, Gacc, Ge, Bt, T, H, D, GA, limite, kid);
     return atencao_back_ws(gom, goE, qm, qE, P, Gacc, Ge, Bt, T, H, D, GA, limite, ws, ws_bytes, false, kid);
 }
 // No reference counterpart: jt_atencao_back_ws without a workspace argument and without any allocation, for callers

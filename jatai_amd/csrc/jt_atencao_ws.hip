@@ -1,9 +1,16 @@
-// Causal ALiBi attention at head width 64 with a caller-provided workspace (the arithmetic of k_atencao_mf: the
-// declared head-width-64 generalization of ops.py:186-258).
+// Causal ALiBi attention at head widths 64, 32 and 16 with a caller-provided workspace (the arithmetic of k_atencao_mf
+// and k_atencao_hd: the declared generalization of ops.py:186-258 to wider heads). HD = 64 spans two 32-dimension
+// halves with an L each; a head of 32 or 16 lies in one block, so one L and one i8 MFMA (K = 32, at 16 half of it
+// zeros) per score tile.
+//
+// Heads of 32 and 16 ran the v_dot2 kernels (jt_atencao_hd.hip), bound by the VALU and by LDS reads: every pair read
+// both operands from LDS and each score was computed three times. Forward + backward at 8 x 512 tokens, 16 heads of
+// 32, BLK 32: 1529 us with them, 144 us here (forward 717 -> 45, backward 768 -> 90 in kernel time); what bounds it
+// now is the per-score VALU work of k_atf (softmax) and the dS bytes that k_atb2 writes and k_atbqkv reads.
 //
 // Forward in two launches:
 //   (1) k_atf_prep, one workgroup per (sequence, head, 64 tokens): the head-wide exponent maxima of q, k, v (one
-//       pass, one reduction), k as m8 << L fragments (int8 [T][64] + L [T][2]) and v aligned as f16 in the order
+//       pass, one reduction), k as m8 << L fragments (int8 [T][HD] + L [T][nl(HD)]) and v aligned as f16 in the order
 //       k_atf's PV MFMAs read it, into the workspace -- converted once instead of once per query block;
 //   (2) k_atf, one workgroup of 4 waves per (sequence, head, 16 query rows): wave w takes the key tiles
 //       t = w, w + 4, ... up to the diagonal. The row maxima and row sums combine across the waves through LDS
@@ -18,9 +25,9 @@
 constexpr size_t cmax_(size_t a, size_t b) { return a > b ? a : b; }
 
 namespace atw {
-// workspace parts, each 256-byte aligned: km8 int8 [BH][T][64]; kl int8 [BH][T][2]; vf f16 [BH][NPV(T)][4][64][8];
-// mx int [BH][4] (emq, emk, emv).
-// km8 rows hold the 8-byte chunks of dimensions 8 k .. 8 k + 7 at chunk 2 (k % 4) + k / 4, so a lane's two MFMA
+// workspace parts, each 256-byte aligned: km8 int8 [BH][T][HD]; kl int8 [BH][T][nl(HD)]; vf f16
+// [BH][NPV(T)][HD / 16][64][8]; mx int [BH][4] (emq, emk, emv).
+// km8 rows at HD = 64 hold the 8-byte chunks of dimensions 8 k .. 8 k + 7 at chunk 2 (k % 4) + k / 4, so a lane's two MFMA
 // fragments of a key (dimensions 8 g .. and 32 + 8 g ..) are one 16-byte load and a wave's 16 keys one kilobyte.
 // vf holds v as the PV MFMAs' B fragments: slot p pairs the key tiles ta = 8 (p / 4) + p % 4 and ta + 4; its
 // block for dimension group dt is 64 lanes x 8 values, lane 16 lg + lr holding dimension 16 dt + lr of the keys
@@ -34,23 +41,24 @@ struct Ws {
 __host__ __device__ inline int npv(int T) { return 4 * ((T / 16 + 7) / 8); }       // slots of vf per head
 __device__ __forceinline__ int pos_k8(int k) { return 2 * (k & 3) + (k >> 2); }     // km8 chunk position of chunk k
 inline size_t alinha256(size_t n) { return (n + 255) & ~(size_t)255; }
-inline size_t bytes_fwd(long long BH, int T) {
+__host__ __device__ constexpr int nl(int hd) { return hd == 64 ? 2 : 1; }           // L values of a token: 32-dim. halves
+inline size_t bytes_fwd(long long BH, int T, int hd) {
     const size_t n = (size_t)BH * T;
-    return alinha256(n * 64) + alinha256(n * 2) + alinha256((size_t)BH * npv(T) * 4096) + alinha256((size_t)BH * 16);
+    return alinha256(n * hd) + alinha256(n * nl(hd)) + alinha256((size_t)BH * npv(T) * 64 * hd) + alinha256((size_t)BH * 16);
 }
-inline Ws parte(void* base, long long BH, int T) {
+inline Ws parte(void* base, long long BH, int T, int hd) {
     const size_t n = (size_t)BH * T;
     char* p = (char*)base;
     Ws w;
-    w.km8 = (int8_t*)p; p += alinha256(n * 64);
-    w.kl = (int8_t*)p; p += alinha256(n * 2);
-    w.vf = (_Float16*)p; p += alinha256((size_t)BH * npv(T) * 4096);
+    w.km8 = (int8_t*)p; p += alinha256(n * hd);
+    w.kl = (int8_t*)p; p += alinha256(n * nl(hd));
+    w.vf = (_Float16*)p; p += alinha256((size_t)BH * npv(T) * 64 * hd);
     w.mx = (int*)p;
     return w;
 }
 // The backward's conversions of q, k, v, written by the forward's conversion pass, which has those values loaded
 // (kept by the caller from the forward to the backward of the same qkv): vm8 int8 [BH][T][64] (chunks as km8's);
-// vL int8 [BH][T][2]; kt, qt f16 [BH][64][T] in fragment order (grava_ft64); mx int [BH][4] (emq, emk, emv: the
+// vL int8 [BH][T][2]; kt, qt f16 [BH][64][T] in fragment order (grava_ft); mx int [BH][4] (emq, emk, emv: the
 // head maxima, before - GA)
 struct Salvo {
     int8_t *vm8, *vL;
@@ -74,25 +82,27 @@ inline Salvo parte_s(void* base, long long BH, int T) {
 }
 }
 
-// Largest block exponent of the 64 / blk blocks of a head slice in one token's exponent row e (column c0): at
-// BLK = 32 the slice's two bytes in one 2-byte load (c0 / 32 is even), at BLK = 128 its one byte.
+// Largest block exponent of the blocks of a head slice in one token's exponent row e (column c0): the two bytes of
+// a head of 64 at BLK = 32 in one 2-byte load (c0 / 32 is even); otherwise the slice lies in one block.
+template <int HD = 64>
 __device__ __forceinline__ int emx_fatia(const int8_t* e, int c0, int blk) {
-    if (blk == 32) {
+    if (HD == 64 && blk == 32) {
         const int x = *reinterpret_cast<const short*>(e + c0 / 32);
         return max((int)(int8_t)x, x >> 8);
     }
     return (int)e[c0 / blk];
 }
 
-// Largest block exponents of three head slices (columns c0 + [0, 64) of E, one per slice) over the T tokens of
+// Largest block exponents of three head slices (columns c0 + [0, HD) of E, one per slice) over the T tokens of
 // sequence b0 / T: one token per thread (T <= 512: at most two), one workgroup reduction (256 threads).
+template <int HD>
 __device__ __forceinline__ void emx3(const int8_t* E, int ld, int ca, int cb, int cc, int blk, int b0, int T, int (&red)[3][4], int& a, int& b,
                                      int& c) {
     const int nbl = ld / blk;
     int ma = SEM_TOPO, mb = SEM_TOPO, mc = SEM_TOPO;
     for (int t = threadIdx.x; t < T; t += 256) {
         const int8_t* e = E + (size_t)(b0 + t) * nbl;
-        ma = max(ma, emx_fatia(e, ca, blk)); mb = max(mb, emx_fatia(e, cb, blk)); mc = max(mc, emx_fatia(e, cc, blk));
+        ma = max(ma, emx_fatia<HD>(e, ca, blk)); mb = max(mb, emx_fatia<HD>(e, cb, blk)); mc = max(mc, emx_fatia<HD>(e, cc, blk));
     }
     ma = g_max<64>(ma); mb = g_max<64>(mb); mc = g_max<64>(mc);
     if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x >> 6] = ma; red[1][threadIdx.x >> 6] = mb; red[2][threadIdx.x >> 6] = mc; }
@@ -102,127 +112,159 @@ __device__ __forceinline__ void emx3(const int8_t* E, int ld, int ca, int cb, in
     c = max(max(red[2][0], red[2][1]), max(red[2][2], red[2][3]));
 }
 
-// The workgroup's 64 tokens x 64 dimensions of a transposed f16 array ([BH][64][T]), staged in LDS by the threads
-// that converted them, written out as 16-byte chunks of each dimension's 128-byte row segment (two per thread)
-// instead of sixteen scattered 2-byte stores per thread. Call after a barrier that follows the tile's writes.
-typedef _Float16 TileT[64][72];                                      // rows padded to 144 bytes (16-byte aligned)
-__device__ __forceinline__ void grava_t64(const TileT& tile, _Float16* __restrict__ cab, int T, int t0) {
+// The workgroup's 64 tokens x HD dimensions of an aligned f16 array, transposed in LDS by the threads that converted
+// them.
+template <int HD> using TileHd = _Float16[HD][72];                   // rows padded to 144 bytes (16-byte aligned)
+// They are written (key tiles 4 p .. 4 p + 3 of a head, p = t0 / 64) in fragment order, the head's [HD][T] f16
+// array as [T / 16 tiles][HD / 16 dt][2 h][16 lr][8]: lane (lr, lg) of an f16 MFMA B fragment reading dimension
+// 16 dt + lr of keys 16 t + 8 h .. + 7 (h = lg % 2) finds them at block (t, dt, h), row lr, so the 32 lanes of one
+// tile read 512 contiguous bytes, where [HD][T] rows gave them 32-byte pieces of 16 rows. Call after a barrier that
+// follows the tile's writes.
+template <int HD>
+__device__ __forceinline__ size_t pos_ft(int t, int dt, int h, int lr) { return ((((size_t)t * (HD / 16) + dt) * 2 + h) * 16 + lr) * 8; }
+template <int HD>
+__device__ __forceinline__ void grava_ft(const TileHd<HD>& tile, _Float16* __restrict__ cab, int t0) {
+    constexpr int ND = HD / 16;
 #pragma unroll
-    for (int x = threadIdx.x; x < 64 * 8; x += 256) {
-        const int row = x >> 3, ch = x & 7;
-        *reinterpret_cast<int4*>(cab + (size_t)row * T + t0 + 8 * ch) = *reinterpret_cast<const int4*>(&tile[row][8 * ch]);
+    for (int y = threadIdx.x; y < 128 * ND; y += 256) {
+        const int h = y / (64 * ND), x = y % (64 * ND), i = x / (16 * ND), dt = (x >> 4) % ND, lr = x & 15, t = t0 / 16 + i;
+        *reinterpret_cast<int4*>(cab + pos_ft<HD>(t, dt, h, lr)) = *reinterpret_cast<const int4*>(&tile[16 * dt + lr][16 * i + 8 * h]);
     }
 }
-// The same 64 tokens x 64 dimensions (key tiles 4 p .. 4 p + 3 of a head, p = t0 / 64) in fragment order, the
-// head's [64][T] f16 array as [T / 16 tiles][4 dt][2 h][16 lr][8]: lane (lr, lg) of an f16 MFMA B fragment reading
-// dimension 16 dt + lr of keys 16 t + 8 h .. + 7 (h = lg % 2) finds them at block (t, dt, h), row lr, so the 32
-// lanes of one tile read 512 contiguous bytes, where [64][T] rows gave them 32-byte pieces of 16 rows.
-__device__ __forceinline__ size_t pos_ft(int t, int dt, int h, int lr) { return ((((size_t)t * 4 + dt) * 2 + h) * 16 + lr) * 8; }
-__device__ __forceinline__ void grava_ft64(const TileT& tile, _Float16* __restrict__ cab, int t0) {
-    const int x = threadIdx.x, i = x >> 6, dt = (x >> 4) & 3, lr = x & 15, t = t0 / 16 + i;
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-        *reinterpret_cast<int4*>(cab + pos_ft(t, dt, h, lr)) = *reinterpret_cast<const int4*>(&tile[16 * dt + lr][16 * i + 8 * h]);
+// HD / 4 consecutive int8 values, the share of one of a token's four conversion threads: one load, and its unpacking
+// (split so that loads can be issued early)
+template <int HD> struct Quarto;
+template <> struct Quarto<64> { typedef int4 T; };
+template <> struct Quarto<32> { typedef int2 T; };
+template <> struct Quarto<16> { typedef int T; };
+template <int HD>
+__device__ __forceinline__ typename Quarto<HD>::T ld_quarto(const int8_t* p) { return *reinterpret_cast<const typename Quarto<HD>::T*>(p); }
+template <int HD>
+__device__ __forceinline__ void abre_quarto(const typename Quarto<HD>::T& x, int (&v)[HD / 4]) {
+    if constexpr (HD == 64) abre_i8(x, v);
+    else le_i8(reinterpret_cast<const int8_t*>(&x), v);
 }
-// 16 m8 values of a token's dimensions 16 c4 .. 16 c4 + 15 into its 64-byte row with the 8-byte chunks k at
+// The m8 values of a token's dimensions HD / 4 c4 .. into its HD-byte row. At HD = 64 the 8-byte chunks k go to
 // 2 (k % 4) + k / 4 (atw::pos_k8), so an MFMA lane's two fragments (dimensions 8 g .. and 32 + 8 g ..) are one
-// 16-byte load
-__device__ __forceinline__ void grava_m8_fragmentos(int8_t* __restrict__ linha, int c4, const int8_t (&m8)[16]) {
-    int8_t lo[8], hi[8];
+// 16-byte load; below, one MFMA takes the whole head and the row keeps its order.
+template <int HD>
+__device__ __forceinline__ void grava_m8_fragmentos(int8_t* __restrict__ linha, int c4, const int8_t (&m8)[HD / 4]) {
+    if constexpr (HD == 64) {
+        int8_t lo[8], hi[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++) { lo[k] = m8[k]; hi[k] = m8[8 + k]; }
-    grava_i8(linha + 8 * atw::pos_k8(2 * c4), lo);
-    grava_i8(linha + 8 * atw::pos_k8(2 * c4 + 1), hi);
+        for (int k = 0; k < 8; k++) { lo[k] = m8[k]; hi[k] = m8[8 + k]; }
+        grava_i8(linha + 8 * atw::pos_k8(2 * c4), lo);
+        grava_i8(linha + 8 * atw::pos_k8(2 * c4 + 1), hi);
+    } else grava_i8(linha + HD / 4 * c4, m8);
 }
-// the two fragments (chunks g and 4 + g) of a row written that way
-__device__ __forceinline__ void le_m8_fragmentos(const int8_t* __restrict__ linha, int g, long& f0, long& f1) {
-    const int4 x = *reinterpret_cast<const int4*>(linha + 16 * g);
-    f0 = (long)(unsigned)x.x | ((long)x.y << 32);
-    f1 = (long)(unsigned)x.z | ((long)x.w << 32);
+// an MFMA lane's fragments of such a row: chunks g and 4 + g (HD = 64), chunk g (HD = 32), chunk g for g < 2 and
+// zeros for the 16 dimensions past the head (HD = 16)
+template <int HD>
+__device__ __forceinline__ void le_m8_fragmentos(const int8_t* __restrict__ linha, int g, long (&f)[atw::nl(HD)]) {
+    if constexpr (HD == 64) {
+        const int4 x = *reinterpret_cast<const int4*>(linha + 16 * g);
+        f[0] = (long)(unsigned)x.x | ((long)x.y << 32);
+        f[1] = (long)(unsigned)x.z | ((long)x.w << 32);
+    } else {
+        f[0] = *reinterpret_cast<const long*>(linha + 8 * (HD == 16 ? g & 1 : g));
+        if (HD == 16 && g >= 2) f[0] = 0;
+    }
+}
+// tile_xyt at head width HD: the two halves' products each shifted by their L, or one product (one block) at 32, 16
+template <int HD>
+__device__ __forceinline__ void tile_hd(const long (&x)[atw::nl(HD)], const long (&y)[atw::nl(HD)], const int (&lx)[4][atw::nl(HD)],
+                                        const int (&ly)[atw::nl(HD)], int (&out)[4]) {
+    if constexpr (HD == 64) tile_xyt(x[0], x[1], y[0], y[1], lx, ly[0], ly[1], out);
+    else {
+        const v4i p = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[0], y[0], v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[v] = shl(p[v], lx[v][0] + ly[0]);
+    }
 }
 
 // SALVA: also the backward's conversions of q, k, v into s (the arithmetic of k_atb_prep's: v as m8 << L
 // fragments, q and k aligned as f16 [64][T], the head maxima), so the backward converts only dO.
-template <bool SALVA = false>
+template <int HD, bool SALVA = false>
 __global__ void __launch_bounds__(256) k_atf_prep(const int8_t* __restrict__ qm, const int8_t* __restrict__ qE, atw::Ws w, atw::Salvo s, int T,
                                                   int H, int D, int blk, int GA) {
-    constexpr int HD = 64;
+    constexpr int ND = HD / 16, CH = HD / 4, NL = atw::nl(HD);
+    static_assert(!SALVA || HD == 64, "the saved conversions are those of head width 64");
     __shared__ int red[3][4];
-    __shared__ __align__(16) TileT tv;
-    __shared__ __align__(16) TileT tqk[SALVA ? 2 : 1];              // SALVA: q and k aligned, for the backward
+    __shared__ __align__(16) TileHd<HD> tv;
+    __shared__ __align__(16) TileHd<HD> tqk[SALVA ? 2 : 1];              // SALVA: q and k aligned, for the backward
     const int nparts = T / 64, bh = blockIdx.x / nparts, part = blockIdx.x % nparts, b = bh / H, h = bh % H;
     const int ld = 3 * D, b0 = b * T, nbl = ld / blk, tid = threadIdx.x;
-    // thread (t, c4): dimensions 16 c4 .. 16 c4 + 15 of token t; its k and v values (and q with SALVA) are loaded
+    // thread (t, c4): dimensions CH c4 .. CH c4 + CH - 1 of token t; its k and v values (and q with SALVA) are loaded
     // before the head maxima's barrier, so their latency overlaps it
-    const int t = part * 64 + (tid >> 2), c4 = tid & 3, half = c4 >> 1;
+    const int t = part * 64 + (tid >> 2), c4 = tid & 3;
     const size_t base = (size_t)(b0 + t) * ld, tt = (size_t)bh * T + t;
-    const int colq = h * HD + 16 * c4, colk = D + colq, colv = 2 * D + colq;
-    const int4 rk = ld16(qm + base + colk), rv = ld16(qm + base + colv);
+    const int colq = h * HD + CH * c4, colk = D + colq, colv = 2 * D + colq;
+    const auto rk = ld_quarto<HD>(qm + base + colk), rv = ld_quarto<HD>(qm + base + colv);
     const int ekt = qE[(size_t)(b0 + t) * nbl + colk / blk], evt = qE[(size_t)(b0 + t) * nbl + colv / blk];
-    int4 rq = make_int4(0, 0, 0, 0);
+    typename Quarto<HD>::T rq{};
     int eqt = 0;
     if constexpr (SALVA) {
-        rq = ld16(qm + base + colq);
+        rq = ld_quarto<HD>(qm + base + colq);
         eqt = qE[(size_t)(b0 + t) * nbl + colq / blk];
     }
     int emq, emk, emv;
-    emx3(qE, ld, h * HD, D + h * HD, 2 * D + h * HD, blk, b0, T, red, emq, emk, emv);
+    emx3<HD>(qE, ld, h * HD, D + h * HD, 2 * D + h * HD, blk, b0, T, red, emq, emk, emv);
     if (part == 0 && tid == 0) {
         w.mx[bh * 4] = emq; w.mx[bh * 4 + 1] = emk; w.mx[bh * 4 + 2] = emv;
         if constexpr (SALVA) { s.mx[bh * 4] = emq; s.mx[bh * 4 + 1] = emk; s.mx[bh * 4 + 2] = emv; }
     }
     {
-        int v[16];
-        abre_i8(rk, v);
+        int v[CH];
+        abre_quarto<HD>(rk, v);
         const int sh = emk - ekt;
-        int8_t m8[16];
+        int8_t m8[CH];
         int L = 0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) { int a; m8_L(v[k], sh, GA, a, L); m8[k] = (int8_t)a; }
-        grava_m8_fragmentos(w.km8 + tt * 64, c4, m8);
-        if ((c4 & 1) == 0) w.kl[tt * 2 + half] = (int8_t)L;
+        for (int k = 0; k < CH; k++) { int a; m8_L(v[k], sh, GA, a, L); m8[k] = (int8_t)a; }
+        grava_m8_fragmentos<HD>(w.km8 + tt * HD, c4, m8);
+        if (c4 % (4 / NL) == 0) w.kl[tt * NL + c4 * NL / 4] = (int8_t)L;
         if constexpr (SALVA) {
             const Desl dk(emk - ekt);
 #pragma unroll
-            for (int k = 0; k < 16; k++) tqk[SALVA ? 1 : 0][16 * c4 + k][tid >> 2] = (_Float16)dk(shl(v[k], GA));
+            for (int k = 0; k < CH; k++) tqk[SALVA ? 1 : 0][CH * c4 + k][tid >> 2] = (_Float16)dk(shl(v[k], GA));
         }
     }
     {
-        int v[16];
-        abre_i8(rv, v);
+        int v[CH];
+        abre_quarto<HD>(rv, v);
         const Desl dv(emv - evt);                                    // rnd(v << GA, emv - evt), one shift per block
 #pragma unroll
-        for (int k = 0; k < 16; k++) tv[16 * c4 + k][tid >> 2] = (_Float16)dv(shl(v[k], GA));
+        for (int k = 0; k < CH; k++) tv[CH * c4 + k][tid >> 2] = (_Float16)dv(shl(v[k], GA));
         if constexpr (SALVA) {
             const int sh = emv - evt;
-            int8_t m8[16];
+            int8_t m8[CH];
             int L = 0;
 #pragma unroll
-            for (int k = 0; k < 16; k++) { int a; m8_L(v[k], sh, GA, a, L); m8[k] = (int8_t)a; }
-            grava_m8_fragmentos(s.vm8 + tt * 64, c4, m8);
-            if ((c4 & 1) == 0) s.vL[tt * 2 + half] = (int8_t)L;
+            for (int k = 0; k < CH; k++) { int a; m8_L(v[k], sh, GA, a, L); m8[k] = (int8_t)a; }
+            grava_m8_fragmentos<HD>(s.vm8 + tt * HD, c4, m8);
+            if (c4 % (4 / NL) == 0) s.vL[tt * NL + c4 * NL / 4] = (int8_t)L;
         }
     }
     if constexpr (SALVA) {
-        int v[16];
-        abre_i8(rq, v);
+        int v[CH];
+        abre_quarto<HD>(rq, v);
         const Desl dq(emq - eqt);
 #pragma unroll
-        for (int k = 0; k < 16; k++) tqk[0][16 * c4 + k][tid >> 2] = (_Float16)dq(shl(v[k], GA));
+        for (int k = 0; k < CH; k++) tqk[0][CH * c4 + k][tid >> 2] = (_Float16)dq(shl(v[k], GA));
     }
     __syncthreads();
-    {   // v fragments of the part's 4 key tiles: thread x writes dimension 16 dt + lr of tile 4 part + x / 64, the
-        // 8-key halves (lg % 2 = 0, 1) of its fragment block
-        const int i = tid >> 6, dt = (tid >> 4) & 3, lr = tid & 15, tk = 4 * part + i;
-        const int slot = 4 * (tk >> 3) + (tk & 3), meio = (tk >> 2) & 1;   // meio 1: the pair's second tile (lg >= 2)
-        _Float16* dst = w.vf + ((((size_t)bh * atw::npv(T) + slot) * 4 + dt) * 64 + 32 * meio + lr) * 8;
+    // v fragments of the part's 4 key tiles: dimension 16 dt + lr of tile 4 part + i, the 8-key halves (lg % 2 = 0, 1)
+    // of its fragment block
 #pragma unroll
-        for (int h2 = 0; h2 < 2; h2++)
-            *reinterpret_cast<int4*>(dst + 16 * 8 * h2) = *reinterpret_cast<const int4*>(&tv[16 * dt + lr][16 * i + 8 * h2]);
+    for (int y = tid; y < 128 * ND; y += 256) {
+        const int h2 = y / (64 * ND), x = y % (64 * ND), i = x / (16 * ND), dt = (x >> 4) % ND, lr = x & 15, tk = 4 * part + i;
+        const int slot = 4 * (tk >> 3) + (tk & 3), meio = (tk >> 2) & 1;   // meio 1: the pair's second tile (lg >= 2)
+        _Float16* dst = w.vf + ((((size_t)bh * atw::npv(T) + slot) * ND + dt) * 64 + 32 * meio + lr) * 8;
+        *reinterpret_cast<int4*>(dst + 16 * 8 * h2) = *reinterpret_cast<const int4*>(&tv[16 * dt + lr][16 * i + 8 * h2]);
     }
     if constexpr (SALVA) {
-        grava_ft64(tqk[0], s.qt + (size_t)bh * 64 * T, part * 64);
-        grava_ft64(tqk[SALVA ? 1 : 0], s.kt + (size_t)bh * 64 * T, part * 64);
+        grava_ft<HD>(tqk[0], s.qt + (size_t)bh * 64 * T, part * 64);
+        grava_ft<HD>(tqk[SALVA ? 1 : 0], s.kt + (size_t)bh * 64 * T, part * 64);
     }
 }
 
@@ -240,13 +282,15 @@ __device__ __forceinline__ void grava_bloco4(const int (&v)[4], int e, int8_t* _
 }
 
 // BLOCO: the output in block format (Oacc, Oe are then the mantissas and exponents, int8) instead of raw
-template <int NTW, bool BLOCO = false>
+template <int HD, int NTW, bool BLOCO = false>
 __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, const int8_t* __restrict__ qE, atw::Ws w, void* __restrict__ Oacc_,
                                              void* __restrict__ Oe_, uint8_t* __restrict__ P, int T, int H, int D, int blk, int GA, int kid) {
-    constexpr int HD = 64, LP = 16 * (NTW + 1);                     // LDS row length of a wave's P (one pad tile)
+    static_assert(!BLOCO || HD == 64, "block outputs: head width 64");
+    constexpr int ND = HD / 16, NL = atw::nl(HD);
+    constexpr int LP = 16 * (NTW + 1);                     // LDS row length of a wave's P (one pad tile)
     __shared__ int sred[4][16];
     __shared__ __align__(16) _Float16 pw[4][16][LP];
-    __shared__ float so[4][16][68];                                  // rows of 68: rows 4 apart fall in other banks
+    __shared__ float so[4][16][HD + 4];                              // padded: rows 4 apart fall in other banks
     __shared__ __align__(16) unsigned short texp[EXP_N];
     static_assert(256 * 2 >= EXP_N / 8 && 256 <= EXP_N / 8, "exp table: one or two chunks per thread");
     int4 tch[2];
@@ -257,65 +301,74 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
     const int b = bh / H, h = bh % H, b0 = b * T;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
     const int eq = w.mx[bh * 4] - GA, ek = w.mx[bh * 4 + 1] - GA, ev = w.mx[bh * 4 + 2] - GA;
-    const int su = -(eq + ek - 3 + 8), incl = 8 - (8 * h) / H;     // log2(64) / 2 = 3
+    const int su = -(eq + ek - ilog2_c(HD) / 2 + 8), incl = 8 - (8 * h) / H;
     const size_t hb = (size_t)bh * T;
     const int ia = 16 * qt + lr, i0 = 16 * qt + 4 * lg;              // A-fragment row; this lane's 4 score rows
     const int nv = qt >= wv ? (qt - wv) / 4 + 1 : 0;                 // this wave's key tiles wv + 4 n, n < nv
     // V fragments of the PV pairs, loaded first (they depend on nothing): pair m, k-index kk = 8 lg + e is key
     // 16 (wv + 4 (2m + kk / 16)) + kk % 16; a pad tile (P = 0 there) reads the wave's first tile of V
     constexpr int NPAR = (NTW + 1) / 2;
-    h8_t vb[NPAR][4];
+    h8_t vb[NPAR][ND];
     // Buffer loads over the head's regions, every one issued (no branch between them): an offset past a region
     // (0x80000000) returns 0 and touches no memory, for a pair or tile the wave does not use and for V past the
     // last key tile (P = 0 and v = 0 there)
-    const auto rsV = __builtin_amdgcn_make_buffer_rsrc((void*)(w.vf + (size_t)bh * atw::npv(T) * 2048), (short)0, atw::npv(T) * 4096, 0x00020000);
-    const auto rsK = __builtin_amdgcn_make_buffer_rsrc((void*)(w.km8 + hb * 64), (short)0, T * 64, 0x00020000);
+    const auto rsV = __builtin_amdgcn_make_buffer_rsrc((void*)(w.vf + (size_t)bh * atw::npv(T) * 32 * HD), (short)0, atw::npv(T) * 64 * HD, 0x00020000);
+    const auto rsK = __builtin_amdgcn_make_buffer_rsrc((void*)(w.km8 + hb * HD), (short)0, T * HD, 0x00020000);
 #pragma unroll
     for (int m = 0; m < NPAR; m++) {                                 // the slot of pair m is 4 m + wv
         const int tv = wv + 4 * (2 * m + (lg >> 1));
-        const int off = 2 * m < nv && tv < nqt ? ((4 * m + wv) * 4 * 64 + lane) * 16 : (int)0x80000000;
+        const int off = 2 * m < nv && tv < nqt ? ((4 * m + wv) * ND * 64 + lane) * 16 : (int)0x80000000;
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
+        for (int dt = 0; dt < ND; dt++) {
             const v4i x = __builtin_amdgcn_raw_buffer_load_b128(rsV, off + dt * 64 * 16, 0, 0);
             vb[m][dt] = __builtin_bit_cast(h8_t, x);
         }
     }
     // K fragments of this wave's key tiles, loaded at entry as well
-    long kb[NTW][2];
-    unsigned lkr[NTW];                                                // both L bytes of a key, split where used
+    long kb[NTW][NL];
+    unsigned lkr[NTW];                                                // the L bytes of a key, split where used
 #pragma unroll
     for (int n = 0; n < NTW; n++) {                                   // a tile the wave does not own: 0 (its L
         const int jl = 16 * (n < nv ? wv + 4 * n : wv) + lr;          // bytes re-read from its first tile)
-        const v4i x = __builtin_amdgcn_raw_buffer_load_b128(rsK, n < nv ? jl * 64 + 16 * lg : (int)0x80000000, 0, 0);
-        kb[n][0] = (long)(unsigned)x[0] | ((long)x[1] << 32);        // le_m8_fragmentos' two fragments
-        kb[n][1] = (long)(unsigned)x[2] | ((long)x[3] << 32);
-        lkr[n] = *reinterpret_cast<const unsigned short*>(w.kl + (hb + jl) * 2);
+        if constexpr (HD == 64) {                                     // le_m8_fragmentos' two fragments
+            const v4i x = __builtin_amdgcn_raw_buffer_load_b128(rsK, n < nv ? jl * 64 + 16 * lg : (int)0x80000000, 0, 0);
+            kb[n][0] = (long)(unsigned)x[0] | ((long)x[1] << 32);
+            kb[n][1] = (long)(unsigned)x[2] | ((long)x[3] << 32);
+            lkr[n] = *reinterpret_cast<const unsigned short*>(w.kl + (hb + jl) * 2);
+        } else {                                                      // HD = 16: 0 past the head's dimensions
+            const bool usa = n < nv && (HD == 32 || lg < 2);
+            kb[n][0] = __builtin_bit_cast(long, __builtin_amdgcn_raw_buffer_load_b64(rsK, usa ? jl * HD + 8 * lg : (int)0x80000000, 0, 0));
+            lkr[n] = (unsigned)(uint8_t)w.kl[hb + jl];
+        }
     }
     // q fragments of the tile's 16 rows, converted here: A row lr = query ia, dimensions 32 c + 8 lg .. + 7
-    __shared__ int qL[16][2];
-    long qa[2];
-    int qv[2][8], qe[2];
+    const int lgq = HD == 16 ? lg & 1 : lg;                           // HD = 16: lanes lg >= 2 hold zeros
+    __shared__ int qL[16][NL];
+    long qa[NL];
+    int qv[NL][8], qe[NL];
 #pragma unroll
-    for (int c = 0; c < 2; c++) {                                     // both halves' loads before either conversion
-        const int col = h * HD + 32 * c + 8 * lg;                     // (m8L_frag's arithmetic)
+    for (int c = 0; c < NL; c++) {                                    // both halves' loads before either conversion
+        const int col = h * HD + 32 * c + 8 * lgq;                    // (m8L_frag's arithmetic)
         le_i8(qm + (size_t)(b0 + ia) * (3 * D) + col, qv[c]);
         qe[c] = qE[(size_t)(b0 + ia) * (3 * D / blk) + col / blk];
     }
     exp_tab_grava(texp, tch);                                        // waits for the table's load only
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < NL; c++) {
         const int s = eq + GA - qe[c];
         int L = 0;
         long pk = 0;
 #pragma unroll
         for (int k = 0; k < 8; k++) { int a; m8_L(qv[c][k], s, GA, a, L); pk |= (long)(uint8_t)a << (8 * k); }
-        qa[c] = pk;
+        qa[c] = HD == 16 && lg >= 2 ? 0 : pk;
         if (lg == 0) qL[lr][c] = L;
     }
     __syncthreads();
-    int lq[4][2];
+    int lq[4][NL];
 #pragma unroll
-    for (int v = 0; v < 4; v++) { lq[v][0] = qL[4 * lg + v][0]; lq[v][1] = qL[4 * lg + v][1]; }
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+        for (int c = 0; c < NL; c++) lq[v][c] = qL[4 * lg + v][c];
     const long long idx = (long long)(b0 + i0) * D + h * HD;
     const Desl dsu(su);                                              // the scores' rounding shift, one per head
     int uu[NTW][4], mx[4] = {U_MIN, U_MIN, U_MIN, U_MIN};
@@ -323,14 +376,15 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
     for (int n = 0; n < NTW; n++) {
         if (n >= nv) continue;                                       // guarded, not break: uu stays in registers
         const int j = 16 * (wv + 4 * n) + lr;
-        const int lk0 = (int)(int8_t)(lkr[n] & 0xff), lk1 = (int)(int8_t)(lkr[n] >> 8);
-        const v4i p0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(qa[0], kb[n][0], v4i{0, 0, 0, 0}, 0, 0, 0);
-        const v4i p1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(qa[1], kb[n][1], v4i{0, 0, 0, 0}, 0, 0, 0);
+        int lk[NL], sc[4];
+#pragma unroll
+        for (int c = 0; c < NL; c++) lk[c] = (int)(int8_t)(lkr[n] >> (8 * c));
+        tile_hd<HD>(qa, kb[n], lq, lk, sc);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int i = i0 + v;
-            const int s = shl(p0[v], lq[v][0] + lk0) + shl(p1[v], lq[v][1] + lk1);
-            const int r = su >= 0 ? dsu(s) : rnd(s, su, kid, idx);
+            // head widths 32, 16: an overflow is reported for causal pairs only, at its row (as k_atencao_hd)
+            const int r = su >= 0 ? dsu(sc[v]) : HD == 64 ? rnd(sc[v], su, kid, idx) : j <= i ? rnd(sc[v], su, kid, idx + (long long)v * D) : 0;
             const int u = j <= i ? r - ((i - j) << incl) : U_MIN;
             uu[n][v] = u;
             mx[v] = max(mx[v], u);
@@ -390,16 +444,16 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
         for (int v = 0; v < 4; v++) pw[wv][4 * lg + v][16 * nv + lr] = (_Float16)0;
     __syncthreads();
     // partial O = P V over this wave's tiles, in pairs
-    f4_t o[4] = {};
+    f4_t o[ND] = {};
 #pragma unroll
     for (int m = 0; m < NPAR; m++) {
         if (2 * m >= nv) continue;
         const h8_t a = *reinterpret_cast<const h8_t*>(&pw[wv][lr][32 * m + 8 * lg]);
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, vb[m][dt], o[dt], 0, 0, 0);
+        for (int dt = 0; dt < ND; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, vb[m][dt], o[dt], 0, 0, 0);
     }
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) so[wv][4 * lg + v][16 * dt + lr] = o[dt][v];
     __syncthreads();
@@ -417,12 +471,12 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
     }
     int* Oacc = (int*)Oacc_;
     int16_t* Oe = (int16_t*)Oe_;
-    // wave wv writes the 16 dimensions 16 wv .. 16 wv + 15
+    // wave wv writes dimensions 16 (wv % ND) .. + 15 of the ND rows 4 lg + ND (wv / ND) ..
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int r = 4 * lg + v, c = 16 * wv + lr;
+    for (int v = 0; v < ND; v++) {
+        const int r = 4 * lg + ND * (wv / ND) + v, c = 16 * (wv % ND) + lr;
         const int ov = (int)(so[0][r][c] + so[1][r][c] + so[2][r][c] + so[3][r][c]);
-        const size_t x = (size_t)(b0 + i0 + v) * D + h * HD + c;
+        const size_t x = (size_t)(b0 + 16 * qt + r) * D + h * HD + c;
         if (ov >= LIM || ov <= -LIM) reporta(E_ACUM, kid, x, ov, -3);
         Oacc[x] = ov;
         Oe[x] = (int16_t)(ev - 8);
@@ -432,7 +486,7 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
 // ---------------------------------------------------------------------------------------------- backward
 // The arithmetic of k_atb_mf_linhas / _gq / _gkv / k_atb_exp, in launches that read converted operands from the
 // workspace and split each 16-row tile's partner tiles over four waves:
-//   (0) k_atb_prep: head maxima of dO, q, k, v; dO, v as m8 << L fragments; k, q, dO aligned as f16 [64][T];
+//   (0) k_atb_prep: head maxima of dO, q, k, v; dO, v as m8 << L fragments; k, q, dO aligned as f16 [HD][T];
 //       for the bound variant (LIMITE), per 64 tokens max |dO| and max ||v||_1 (ops.py:231-235); or k_atb_prep_s,
 //       the same for dO alone when the forward's conversion pass saved those of q, k, v (exact variant);
 //   (1) k_atb1 (exact variant): per query tile, max |gP| over its causal pairs;
@@ -445,8 +499,8 @@ __global__ void __launch_bounds__(256) k_atf(const int8_t* __restrict__ qm, cons
 namespace atw {
 constexpr int SLOTS = 32;            // per head and kind: T / 16 <= 32 query tiles
 struct WsB {
-    int8_t *gm8, *gL, *vm8, *vL;     // dO, v: m8 [BH][T][64] (chunks as km8's), L [BH][T][2]
-    _Float16 *kt, *qt, *gt;          // k, q, dO aligned: f16 [BH][64][T] in fragment order (grava_ft64)
+    int8_t *gm8, *gL, *vm8, *vL;     // dO, v: m8 [BH][T][HD] (chunks as km8's), L [BH][T][nl(HD)]
+    _Float16 *kt, *qt, *gt;          // k, q, dO aligned: f16 [BH][HD][T] in fragment order (grava_ft)
     int* sl;                         // s_i [BH][T]
     int* mx;                         // [BH][4]: ego, eq, ek, ev (head maxima - GA)
     int* p1a;                        // [BH][SLOTS]: max |gP| per query tile, or max |dO| per 64 tokens (LIMITE)
@@ -457,22 +511,22 @@ struct WsB {
 // element (i, j) of head bh's dS before its shrink (|value| < 2^25: P <= 255, |gP' - s| < 2^17), in tile (i/16, j/16)
 // at row i % 16, column j % 16; written by k_atb2 for the causal tiles, read by k_atbqkv
 __device__ __forceinline__ size_t ds_pos(int bh, int nqt, int qt, int kt) { return (((size_t)bh * nqt + qt) * nqt + kt) * 256; }
-inline size_t bytes_back(long long BH, int T) {
+inline size_t bytes_back(long long BH, int T, int hd) {
     const size_t n = (size_t)BH * T;
-    return 2 * (alinha256(n * 64) + alinha256(n * 2)) + 3 * alinha256(n * 64 * 2) + alinha256(n * 4) + alinha256((size_t)BH * 16) +
+    return 2 * (alinha256(n * hd) + alinha256(n * nl(hd))) + 3 * alinha256(n * hd * 2) + alinha256(n * 4) + alinha256((size_t)BH * 16) +
            5 * alinha256((size_t)BH * SLOTS * 4) + alinha256((size_t)BH * T * T * 4);
 }
-inline WsB parte_b(void* base, long long BH, int T) {
+inline WsB parte_b(void* base, long long BH, int T, int hd) {
     const size_t n = (size_t)BH * T;
     char* p = (char*)base;
     WsB w;
-    w.gm8 = (int8_t*)p; p += alinha256(n * 64);
-    w.gL = (int8_t*)p; p += alinha256(n * 2);
-    w.vm8 = (int8_t*)p; p += alinha256(n * 64);
-    w.vL = (int8_t*)p; p += alinha256(n * 2);
-    w.kt = (_Float16*)p; p += alinha256(n * 64 * 2);
-    w.qt = (_Float16*)p; p += alinha256(n * 64 * 2);
-    w.gt = (_Float16*)p; p += alinha256(n * 64 * 2);
+    w.gm8 = (int8_t*)p; p += alinha256(n * hd);
+    w.gL = (int8_t*)p; p += alinha256(n * nl(hd));
+    w.vm8 = (int8_t*)p; p += alinha256(n * hd);
+    w.vL = (int8_t*)p; p += alinha256(n * nl(hd));
+    w.kt = (_Float16*)p; p += alinha256(n * hd * 2);
+    w.qt = (_Float16*)p; p += alinha256(n * hd * 2);
+    w.gt = (_Float16*)p; p += alinha256(n * hd * 2);
     w.sl = (int*)p; p += alinha256(n * 4);
     w.mx = (int*)p; p += alinha256((size_t)BH * 16);
     w.p1a = (int*)p; p += alinha256((size_t)BH * SLOTS * 4);
@@ -525,7 +579,7 @@ __device__ __forceinline__ void atb_gp(const int8_t* __restrict__ gom, const int
                                        const int8_t* __restrict__ qE, atw::WsB& w, int T, int H, int D, int blk, int GA, int BH,
                                        int8_t* lds, int (&red)[4][4]) {
     constexpr int HD = 64, RS = 72;
-    static_assert(3 * sizeof(TileT) >= 256 * RS + 64 * RS + 128 + 512, "atb_gp's LDS fits k_atb_prep's tiles");
+    static_assert(3 * sizeof(TileHd<HD>) >= 256 * RS + 64 * RS + 128 + 512, "atb_gp's LDS fits k_atb_prep's tiles");
     const int bh = (int)blockIdx.x % BH, g = (int)blockIdx.x / BH, b = bh / H, h = bh % H;
     const int ld = 3 * D, b0 = b * T, tid = threadIdx.x, nbl = ld / blk, nbg = D / blk, nqt = T / 16;
     const int c4 = tid & 3, half = c4 >> 1, tl = tid >> 2, colg = h * HD + 16 * c4;
@@ -653,18 +707,18 @@ __device__ __forceinline__ void atb_gp(const int8_t* __restrict__ gom, const int
     }
 }
 
-template <int LIMITE, bool GP = false>
+template <int HD, int LIMITE, bool GP = false>
 __global__ void __launch_bounds__(256) k_atb_prep(const int8_t* __restrict__ gom, const int8_t* __restrict__ goE, const int8_t* __restrict__ qm,
                                                   const int8_t* __restrict__ qE, atw::WsB w, int T, int H, int D, int blk, int GA) {
-    constexpr int HD = 64;
+    constexpr int CH = HD / 4, NL = atw::nl(HD);
     __shared__ int red[4][4];
     __shared__ int red1[4];
-    __shared__ __align__(16) TileT tiles[3];                         // dO, q, k; or atb_gp's fragments (23.7 KB)
-    TileT &tg = tiles[0], &tq = tiles[1], &tk = tiles[2];
+    __shared__ __align__(16) TileHd<HD> tiles[3];                         // dO, q, k; or atb_gp's fragments (23.7 KB)
+    TileHd<HD> &tg = tiles[0], &tq = tiles[1], &tk = tiles[2];
     const int nparts = T / 64;
     int wg = (int)blockIdx.x;
     if constexpr (GP) {
-        static_assert(LIMITE == 0, "per-tile max |gP| belongs to the exact variant");
+        static_assert(LIMITE == 0 && HD == 64, "per-tile max |gP| in this launch: the exact variant at head width 64");
         const int BH = (int)gridDim.x / (2 * nparts);
         if (wg < BH * nparts) {                                        // uniform per workgroup
             atb_gp<LIMITE>(gom, goE, qm, qE, w, T, H, D, blk, GA, BH, reinterpret_cast<int8_t*>(&tiles[0][0][0]), red);
@@ -674,13 +728,13 @@ __global__ void __launch_bounds__(256) k_atb_prep(const int8_t* __restrict__ gom
     }
     const int bh = wg / nparts, part = wg % nparts, b = bh / H, h = bh % H;
     const int ld = 3 * D, b0 = b * T, tid = threadIdx.x, nbl = ld / blk, nbg = D / blk;
-    // thread (t, c4): dimensions 16 c4 .. 16 c4 + 15 of token t. Every value it converts is loaded first, so the
+    // thread (t, c4): dimensions CH c4 .. CH c4 + CH - 1 of token t. Every value it converts is loaded first, so the
     // loads overlap the head maxima's reduction below.
-    const int t = part * 64 + (tid >> 2), c4 = tid & 3, half = c4 >> 1;
+    const int t = part * 64 + (tid >> 2), c4 = tid & 3;
     const size_t tt = (size_t)bh * T + t, lq = (size_t)(b0 + t) * ld;
-    const int colg = h * HD + 16 * c4;
-    const int4 rg = ld16(gom + (size_t)(b0 + t) * D + colg), rv = ld16(qm + lq + 2 * D + colg);
-    const int4 rq = ld16(qm + lq + colg), rk = ld16(qm + lq + D + colg);
+    const int colg = h * HD + CH * c4;
+    const auto rg = ld_quarto<HD>(gom + (size_t)(b0 + t) * D + colg), rv = ld_quarto<HD>(qm + lq + 2 * D + colg);
+    const auto rq = ld_quarto<HD>(qm + lq + colg), rk = ld_quarto<HD>(qm + lq + D + colg);
     const int egt = goE[(size_t)(b0 + t) * nbg + colg / blk], evt = qE[(size_t)(b0 + t) * nbl + (2 * D + colg) / blk];
     const int eqt = qE[(size_t)(b0 + t) * nbl + colg / blk], ekt = qE[(size_t)(b0 + t) * nbl + (D + colg) / blk];
     // head maxima of the q, k, v and dO exponents in one reduction
@@ -689,10 +743,10 @@ __global__ void __launch_bounds__(256) k_atb_prep(const int8_t* __restrict__ gom
         int m[4] = {SEM_TOPO, SEM_TOPO, SEM_TOPO, SEM_TOPO};
         for (int tk = tid; tk < T; tk += 256) {                      // one token per thread (T <= 512: at most two)
             const int8_t* e = qE + (size_t)(b0 + tk) * nbl;
-            m[0] = max(m[0], emx_fatia(e, h * HD, blk));
-            m[1] = max(m[1], emx_fatia(e, D + h * HD, blk));
-            m[2] = max(m[2], emx_fatia(e, 2 * D + h * HD, blk));
-            m[3] = max(m[3], emx_fatia(goE + (size_t)(b0 + tk) * nbg, h * HD, blk));
+            m[0] = max(m[0], emx_fatia<HD>(e, h * HD, blk));
+            m[1] = max(m[1], emx_fatia<HD>(e, D + h * HD, blk));
+            m[2] = max(m[2], emx_fatia<HD>(e, 2 * D + h * HD, blk));
+            m[3] = max(m[3], emx_fatia<HD>(goE + (size_t)(b0 + tk) * nbg, h * HD, blk));
         }
 #pragma unroll
         for (int x = 0; x < 4; x++) m[x] = g_max<64>(m[x]);
@@ -708,50 +762,50 @@ __global__ void __launch_bounds__(256) k_atb_prep(const int8_t* __restrict__ gom
     if (part == 0 && tid == 0) { w.mx[bh * 4] = emg - GA; w.mx[bh * 4 + 1] = emq - GA; w.mx[bh * 4 + 2] = emk - GA; w.mx[bh * 4 + 3] = emv - GA; }
     int amax = 0, v1 = 0;
     {   // dO: m8 << L fragments and aligned f16
-        int v[16];
-        abre_i8(rg, v);
+        int v[CH];
+        abre_quarto<HD>(rg, v);
         const int s = emg - egt;
         const Desl ds(s);
-        int8_t m8[16];
+        int8_t m8[CH];
         int L = 0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
+        for (int k = 0; k < CH; k++) {
             int a; m8_L(v[k], s, GA, a, L); m8[k] = (int8_t)a;
             const int al = ds(shl(v[k], GA));
             amax = max(amax, abs(al));
-            tg[16 * c4 + k][tid >> 2] = (_Float16)al;
+            tg[CH * c4 + k][tid >> 2] = (_Float16)al;
         }
-        grava_m8_fragmentos(w.gm8 + tt * 64, c4, m8);
-        if ((c4 & 1) == 0) w.gL[tt * 2 + half] = (int8_t)L;
+        grava_m8_fragmentos<HD>(w.gm8 + tt * HD, c4, m8);
+        if (c4 % (4 / NL) == 0) w.gL[tt * NL + c4 * NL / 4] = (int8_t)L;
     }
     {   // v: m8 << L fragments (and ||v||_1 for LIMITE)
-        int v[16];
-        abre_i8(rv, v);
+        int v[CH];
+        abre_quarto<HD>(rv, v);
         const int s = emv - evt;
         const Desl ds(s);
-        int8_t m8[16];
+        int8_t m8[CH];
         int L = 0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
+        for (int k = 0; k < CH; k++) {
             int a; m8_L(v[k], s, GA, a, L); m8[k] = (int8_t)a;
             if (LIMITE) v1 += abs(ds(shl(v[k], GA)));
         }
-        grava_m8_fragmentos(w.vm8 + tt * 64, c4, m8);
-        if ((c4 & 1) == 0) w.vL[tt * 2 + half] = (int8_t)L;
+        grava_m8_fragmentos<HD>(w.vm8 + tt * HD, c4, m8);
+        if (c4 % (4 / NL) == 0) w.vL[tt * NL + c4 * NL / 4] = (int8_t)L;
     }
 #pragma unroll
     for (int x = 0; x < 2; x++) {   // q (x = 0), k (x = 1): aligned f16, transposed
-        int v[16];
-        abre_i8(x ? rk : rq, v);
+        int v[CH];
+        abre_quarto<HD>(x ? rk : rq, v);
         const Desl ds((x ? emk : emq) - (x ? ekt : eqt));
-        TileT& dst = x ? tk : tq;
+        TileHd<HD>& dst = x ? tk : tq;
 #pragma unroll
-        for (int k = 0; k < 16; k++) dst[16 * c4 + k][tid >> 2] = (_Float16)ds(shl(v[k], GA));
+        for (int k = 0; k < CH; k++) dst[CH * c4 + k][tid >> 2] = (_Float16)ds(shl(v[k], GA));
     }
     __syncthreads();
-    grava_ft64(tg, w.gt + (size_t)bh * 64 * T, part * 64);
-    grava_ft64(tq, w.qt + (size_t)bh * 64 * T, part * 64);
-    grava_ft64(tk, w.kt + (size_t)bh * 64 * T, part * 64);
+    grava_ft<HD>(tg, w.gt + (size_t)bh * HD * T, part * 64);
+    grava_ft<HD>(tq, w.qt + (size_t)bh * HD * T, part * 64);
+    grava_ft<HD>(tk, w.kt + (size_t)bh * HD * T, part * 64);
     if (LIMITE) {
         v1 = quad_soma(v1);
         const int a = wg_max4(amax, red1), c = wg_max4(v1, red1);
@@ -766,7 +820,7 @@ __global__ void __launch_bounds__(256) k_atb_prep_s(const int8_t* __restrict__ g
                                                     const int* __restrict__ smx, int T, int H, int D, int blk, int GA) {
     constexpr int HD = 64;
     __shared__ int red[4];
-    __shared__ __align__(16) TileT tg;
+    __shared__ __align__(16) TileHd<HD> tg;
     const int nparts = T / 64, bh = blockIdx.x / nparts, part = blockIdx.x % nparts, b = bh / H, h = bh % H;
     const int b0 = b * T, tid = threadIdx.x, nbg = D / blk;
     const int t = part * 64 + (tid >> 2), c4 = tid & 3, half = c4 >> 1;
@@ -796,31 +850,40 @@ __global__ void __launch_bounds__(256) k_atb_prep_s(const int8_t* __restrict__ g
             int a; m8_L(v[k], s, GA, a, L); m8[k] = (int8_t)a;
             tg[16 * c4 + k][tid >> 2] = (_Float16)ds(shl(v[k], GA));
         }
-        grava_m8_fragmentos(w.gm8 + tt * 64, c4, m8);
+        grava_m8_fragmentos<HD>(w.gm8 + tt * 64, c4, m8);
         if ((c4 & 1) == 0) w.gL[tt * 2 + half] = (int8_t)L;
     }
     __syncthreads();
-    grava_ft64(tg, w.gt + (size_t)bh * 64 * T, part * 64);
+    grava_ft<HD>(tg, w.gt + (size_t)bh * 64 * T, part * 64);
 }
 
 // gP tile of query rows i0 .. i0 + 3 (this lane) x key j = 16 t + lr from the workspace fragments
-struct FragQ {                                      // dO fragments of a query tile (A operand) and their L
-    long ga[2];
-    int lx[4][2];
+template <int HD> struct FragQ {                    // dO fragments of a query tile (A operand) and their L
+    long ga[atw::nl(HD)];
+    int lx[4][atw::nl(HD)];
 };
-__device__ __forceinline__ FragQ frag_q(const atw::WsB& w, size_t hb, int qt, int lr, int lg) {
-    FragQ f;
+template <int HD>
+__device__ __forceinline__ FragQ<HD> frag_q(const atw::WsB& w, size_t hb, int qt, int lr, int lg) {
+    constexpr int NL = atw::nl(HD);
+    FragQ<HD> f;
     const size_t ia = hb + 16 * qt + lr, i0 = hb + 16 * qt + 4 * lg;
-    le_m8_fragmentos(w.gm8 + ia * 64, lg, f.ga[0], f.ga[1]);
+    le_m8_fragmentos<HD>(w.gm8 + ia * HD, lg, f.ga);
 #pragma unroll
-    for (int v = 0; v < 4; v++) { f.lx[v][0] = w.gL[(i0 + v) * 2]; f.lx[v][1] = w.gL[(i0 + v) * 2 + 1]; }
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+        for (int c = 0; c < NL; c++) f.lx[v][c] = w.gL[(i0 + v) * NL + c];
     return f;
 }
-__device__ __forceinline__ void gp_tile(const atw::WsB& w, size_t hb, const FragQ& f, int t, int lr, int lg, int (&o)[4]) {
+template <int HD>
+__device__ __forceinline__ void gp_tile(const atw::WsB& w, size_t hb, const FragQ<HD>& f, int t, int lr, int lg, int (&o)[4]) {
+    constexpr int NL = atw::nl(HD);
     const size_t j = hb + 16 * t + lr;
-    long v0, v1;
-    le_m8_fragmentos(w.vm8 + j * 64, lg, v0, v1);
-    tile_xyt(f.ga[0], f.ga[1], v0, v1, f.lx, w.vL[j * 2], w.vL[j * 2 + 1], o);
+    long vf[NL];
+    int lv[NL];
+    le_m8_fragmentos<HD>(w.vm8 + j * HD, lg, vf);
+#pragma unroll
+    for (int c = 0; c < NL; c++) lv[c] = w.vL[j * NL + c];
+    tile_hd<HD>(f.ga, vf, f.lx, lv, o);
 }
 // query tile of this workgroup, in decreasing work across all heads (tile qt pairs with qt + 1 key tiles)
 #define ATB_TILE_Q ATB_TILE_Q_(blockIdx.x, gridDim.x)
@@ -831,19 +894,19 @@ __device__ __forceinline__ void gp_tile(const atw::WsB& w, size_t hb, const Frag
     const size_t hb = (size_t)bh * T;                                                                                  \
     const int i0 = 16 * qt + 4 * lg, nv = qt >= wv ? (qt - wv) / 4 + 1 : 0;
 
-template <int NTW>
+template <int HD, int NTW>
 __global__ void __launch_bounds__(256) k_atb1(atw::WsB w, int T, int H) {
     __shared__ int red[4];
     ATB_TILE_Q
     (void)b0;
-    const FragQ f = frag_q(w, hb, qt, lr, lg);
+    const FragQ<HD> f = frag_q<HD>(w, hb, qt, lr, lg);
     int mg = 0;
 #pragma unroll
     for (int n = 0; n < NTW; n++) {
         if (n >= nv) continue;
         const int t = wv + 4 * n, j = 16 * t + lr;
         int o[4];
-        gp_tile(w, hb, f, t, lr, lg, o);
+        gp_tile<HD>(w, hb, f, t, lr, lg, o);
 #pragma unroll
         for (int v = 0; v < 4; v++) if (j <= i0 + v) mg = max(mg, abs(o[v]));
     }
@@ -851,12 +914,12 @@ __global__ void __launch_bounds__(256) k_atb1(atw::WsB w, int T, int H) {
     if (tid == 0) w.p1a[bh * atw::SLOTS + qt] = mg;
 }
 
-template <int NTW, int LIMITE>
+template <int HD, int NTW, int LIMITE>
 __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restrict__ P, int T, int H, int D, int kid) {
     __shared__ int red[4];
     __shared__ int sred[4][16];
     ATB_TILE_Q
-    const FragQ f = frag_q(w, hb, qt, lr, lg);
+    const FragQ<HD> f = frag_q<HD>(w, hb, qt, lr, lg);
     const int sh = atw::sh_gp_ws<LIMITE>(w, bh, T);                  // after frag_q's loads are issued
     const Desl dsh(sh);                                              // gP's shrink, one shift per head
     const uint8_t* Pb = P + (size_t)bh * T * T;
@@ -868,8 +931,9 @@ __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restr
         if (n >= nv) continue;
         const int t = wv + 4 * n, j = 16 * t + lr;
         int o[4];
-        gp_tile(w, hb, f, t, lr, lg, o);
+        gp_tile<HD>(w, hb, f, t, lr, lg, o);
         pr[n] = *reinterpret_cast<const unsigned*>(Pb + (size_t)j * T + i0);     // P_ij, rows i0 .. i0 + 3
+        if (HD != 64 && t == qt) pr[n] &= j <= i0 ? ~0u : j - i0 > 3 ? 0u : ~0u << (8 * (j - i0));   // causal bytes only
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int xv = j <= i0 + v ? dsh(o[v]) : 0;
@@ -890,7 +954,7 @@ __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restr
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int tot = sred[0][4 * lg + v] + sred[1][4 * lg + v] + sred[2][4 * lg + v] + sred[3][4 * lg + v];
-        if ((tot >= LIM || tot <= -LIM) && lr == 0 && wv == 0) reporta(E_ACUM, kid, (long long)(b0 + i0 + v) * ld + h * 64, tot, -4);
+        if ((tot >= LIM || tot <= -LIM) && lr == 0 && wv == 0) reporta(E_ACUM, kid, (long long)(b0 + i0 + v) * ld + h * HD, tot, -4);
         sl[v] = rnd_d(tot, 8);
         if (lr == 0 && wv == 0) w.sl[hb + i0 + v] = sl[v];
     }
@@ -918,19 +982,22 @@ __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restr
     }
 }
 
-// sums the four waves' partials parc[w][16][64] (this lane: rows 4 lg + v, column 16 dt + lr of wave wv's
-// registers) -- written by every wave, then wave wv adds column group 16 wv .. 16 wv + 15 -- into out[v]. The sums
-// are the exact integer results of at most 256 products |dS| |k| <= 4096 * 2032 (or P |dO| <= 255 * 2032), below
-// 2^31: 32-bit adds (modular, unsigned) give them exactly, as the int64 sums of the arithmetic would.
-__device__ __forceinline__ void soma_ondas(int (&parc)[4][16][64], const int (&mine)[4][4], int wv, int lr, int lg, int (&out)[4]) {
+// sums the four waves' partials parc[w][16][HD] (this lane: rows 4 lg + v, column 16 dt + lr of wave wv's
+// registers) -- written by every wave, then wave wv adds the column group 16 (wv % ND) .. + 15 of the ND = HD / 16
+// rows 4 lg + ND (wv / ND) + v -- into out[v]. The sums are the exact integer results of products |dS| |k| <=
+// 4096 * 2032 (T <= 256) or 1024 * 2032 (T = 512), or P |dO| <= 255 * 2032, below 2^31: 32-bit adds (modular,
+// unsigned) give them exactly, as the int64 sums of the arithmetic would.
+template <int HD>
+__device__ __forceinline__ void soma_ondas(int (&parc)[4][16][HD], const int (&mine)[HD / 16][4], int wv, int lr, int lg, int (&out)[HD / 16]) {
+    constexpr int ND = HD / 16;
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) parc[wv][4 * lg + v][16 * dt + lr] = mine[dt][v];
     __syncthreads();
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int r = 4 * lg + v, c = 16 * wv + lr;
+    for (int v = 0; v < ND; v++) {
+        const int r = 4 * lg + ND * (wv / ND) + v, c = 16 * (wv % ND) + lr;
         out[v] = (int)((unsigned)parc[0][r][c] + (unsigned)parc[1][r][c] + (unsigned)parc[2][r][c] + (unsigned)parc[3][r][c]);
     }
     __syncthreads();
@@ -952,12 +1019,13 @@ __device__ __forceinline__ void soma_ondas_bloco(int (&parc)[4][16][64], const i
 
 // gq of workgroup blk of nblk. lds: dS tiles, then (after a barrier) the waves' 32-bit partial sums in the same
 // LDS (LDS_ATBQKV bytes).
-template <int NTW, int LIMITE, bool BLOCO = false>
+template <int HD, int NTW, int LIMITE, bool BLOCO = false>
 __device__ __forceinline__ void atbq_corpo(const atw::WsB& w, const uint8_t* __restrict__ P, int* __restrict__ Gacc, int16_t* __restrict__ Ge,
                                            int T, int H, int D, int dsb, int kid, char* lds, const int blk, const int nblk) {
-    constexpr int LP = 16 * (NTW + 1);
+    static_assert(!BLOCO || HD == 64, "block outputs: head width 64");
+    constexpr int LP = 16 * (NTW + 1), ND = HD / 16;
     auto dw = reinterpret_cast<short (*)[16][LP]>(lds);
-    auto& parc = *reinterpret_cast<int (*)[4][16][64]>(lds);
+    auto& parc = *reinterpret_cast<int (*)[4][16][HD]>(lds);
     ATB_TILE_Q_(blk, nblk)
     (void)P;
     // dS before its shrink, as k_atb2 stored it (0 past the diagonal): rows 4 lg + v of tile (qt, t), column lr
@@ -985,7 +1053,7 @@ __device__ __forceinline__ void atbq_corpo(const atw::WsB& w, const uint8_t* __r
         for (int v = 0; v < 4; v++) dw[wv][4 * lg + v][16 * nv + lr] = 0;
     __syncthreads();
     // gq partial = dS K over this wave's key tiles, in pairs; dS = a 256 + b 16 + c (see the MFMA backward above)
-    f4_t acc[4][3] = {};
+    f4_t acc[ND][3] = {};
 #pragma unroll
     for (int m = 0; m < (NTW + 1) / 2; m++) {
         if (2 * m >= nv) continue;
@@ -994,37 +1062,39 @@ __device__ __forceinline__ void atbq_corpo(const atw::WsB& w, const uint8_t* __r
         int tk = wv + 4 * (2 * m + (lg >> 1));
         if (tk >= nqt) tk = wv;                                      // pad tile: dS = 0 there
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
-            const h8_t kv = *reinterpret_cast<const h8_t*>(w.kt + (size_t)bh * 64 * T + pos_ft(tk, dt, lg & 1, lr));
+        for (int dt = 0; dt < ND; dt++) {
+            const h8_t kv = *reinterpret_cast<const h8_t*>(w.kt + (size_t)bh * HD * T + pos_ft<HD>(tk, dt, lg & 1, lr));
             acc[dt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, kv, acc[dt][0], 0, 0, 0);
             acc[dt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pb, kv, acc[dt][1], 0, 0, 0);
             acc[dt][2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pc, kv, acc[dt][2], 0, 0, 0);
         }
     }
-    int mine[4][4], gq[4];
+    int mine[ND][4];
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) mine[dt][v] = junta3(acc[dt][0][v], acc[dt][1][v], acc[dt][2][v]);
     const int ld = 3 * D;
     __syncthreads();                                                 // every wave is done with dw: parc reuses it
     if constexpr (BLOCO) {                                           // Gacc, Ge: int8 mantissas and exponents
+        int gq[4];
         soma_ondas_bloco(parc, mine, wv, lr, lg, gq);
         const int r = tid >> 4, c = 4 * (tid & 15);
-        const size_t x = (size_t)(b0 + 16 * qt + r) * ld + h * 64 + c;
+        const size_t x = (size_t)(b0 + 16 * qt + r) * ld + h * HD + c;
         int g4[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             if (gq[k] >= LIM || gq[k] <= -LIM) reporta(E_ACUM, kid, x + k, gq[k], -5);
             g4[k] = (int)gq[k];
         }
-        grava_bloco4(g4, eds + ek, (int8_t*)Gacc, (int8_t*)Ge, x, (size_t)(b0 + 16 * qt + r) * (ld / 32) + (h * 64 + c) / 32, kid);
+        grava_bloco4(g4, eds + ek, (int8_t*)Gacc, (int8_t*)Ge, x, (size_t)(b0 + 16 * qt + r) * (ld / 32) + (h * HD + c) / 32, kid);
         return;
     }
-    soma_ondas(parc, mine, wv, lr, lg, gq);
+    int gq[ND];
+    soma_ondas<HD>(parc, mine, wv, lr, lg, gq);
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const size_t o = (size_t)(b0 + i0 + v) * ld + h * 64 + 16 * wv + lr;
+    for (int v = 0; v < ND; v++) {
+        const size_t o = (size_t)(b0 + i0 + ND * (wv / ND) + v) * ld + h * HD + 16 * (wv % ND) + lr;
         if (gq[v] >= LIM || gq[v] <= -LIM) reporta(E_ACUM, kid, o, gq[v], -5);
         Gacc[o] = (int)gq[v];
         Ge[o] = (int16_t)(eds + ek);
@@ -1033,14 +1103,15 @@ __device__ __forceinline__ void atbq_corpo(const atw::WsB& w, const uint8_t* __r
 
 // gk, gv of workgroup blk of nblk. lds: dS and P tiles, then (after a barrier) the waves' 32-bit partial sums in
 // the same LDS (LDS_ATBQKV bytes).
-template <int NTW> constexpr size_t LDS_ATBQKV = cmax_(sizeof(short) * 4 * 16 * 16 * (NTW + 1) + 4 * 16 * 16 * (NTW + 1), sizeof(int) * 4 * 16 * 64);
-template <int NTW, int LIMITE, bool BLOCO = false>
+template <int HD, int NTW> constexpr size_t LDS_ATBQKV = cmax_(sizeof(short) * 4 * 16 * 16 * (NTW + 1) + 4 * 16 * 16 * (NTW + 1), sizeof(int) * 4 * 16 * HD);
+template <int HD, int NTW, int LIMITE, bool BLOCO = false>
 __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __restrict__ P, int* __restrict__ Gacc, int16_t* __restrict__ Ge,
                                             int T, int H, int D, int dsb, int kid, char* lds, const int blk, const int nblk) {
-    constexpr int LP = 16 * (NTW + 1);
+    static_assert(!BLOCO || HD == 64, "block outputs: head width 64");
+    constexpr int LP = 16 * (NTW + 1), ND = HD / 16;
     auto dw = reinterpret_cast<short (*)[16][LP]>(lds);
     auto pw = reinterpret_cast<uint8_t (*)[16][LP]>(lds + sizeof(short) * 4 * 16 * LP);
-    auto& parc = *reinterpret_cast<int (*)[4][16][64]>(lds);
+    auto& parc = *reinterpret_cast<int (*)[4][16][HD]>(lds);
     // key tile kt pairs with the query tiles kt .. nqt - 1: decreasing work is increasing kt
     const int nqt = T / 16, BH = nblk / nqt, bh = blk % BH, kt = (int)(blk / BH);
     const int b = bh / H, h = bh % H, b0 = b * T;
@@ -1099,7 +1170,7 @@ __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __
 #pragma unroll
         for (int v = 0; v < 4; v++) { dw[wv][4 * lg + v][16 * nv + lr] = 0; pw[wv][4 * lg + v][16 * nv + lr] = 0; }
     __syncthreads();
-    f4_t ak[4][3] = {}, av[4][2] = {};
+    f4_t ak[ND][3] = {}, av[ND][2] = {};
 #pragma unroll
     for (int m = 0; m < (NTW + 1) / 2; m++) {
         if (2 * m >= nv) continue;
@@ -1111,8 +1182,8 @@ __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __
         int tq = kt + wv + 4 * (2 * m + (lg >> 1));
         if (tq >= nqt) tq = kt + wv;                                 // pad tile: dS = P = 0 there
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) {
-            const size_t r = (size_t)bh * 64 * T + pos_ft(tq, dt, lg & 1, lr);
+        for (int dt = 0; dt < ND; dt++) {
+            const size_t r = (size_t)bh * HD * T + pos_ft<HD>(tq, dt, lg & 1, lr);
             const h8_t qv = *reinterpret_cast<const h8_t*>(w.qt + r);
             const h8_t gv = *reinterpret_cast<const h8_t*>(w.gt + r);
             ak[dt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa, qv, ak[dt][0], 0, 0, 0);
@@ -1122,22 +1193,23 @@ __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __
             av[dt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, gv, av[dt][1], 0, 0, 0);
         }
     }
-    int mine[4][4], gk[4], gvv[4];
+    int mine[ND][4];
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) mine[dt][v] = junta3(ak[dt][0][v], ak[dt][1][v], ak[dt][2][v]);
     const int ld = 3 * D;
     __syncthreads();                                                 // every wave is done with dw, pw: parc reuses them
     if constexpr (BLOCO) {                                           // Gacc, Ge: int8 mantissas and exponents
+        int gk[4], gvv[4];
         soma_ondas_bloco(parc, mine, wv, lr, lg, gk);
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++)
+        for (int dt = 0; dt < ND; dt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) mine[dt][v] = junta2(av[dt][0][v], av[dt][1][v]);
         soma_ondas_bloco(parc, mine, wv, lr, lg, gvv);
         const int r = tid >> 4, c = 4 * (tid & 15);
-        const size_t x = (size_t)(b0 + 16 * kt + r) * ld + h * 64 + c, xe = (size_t)(b0 + 16 * kt + r) * (ld / 32) + (h * 64 + c) / 32;
+        const size_t x = (size_t)(b0 + 16 * kt + r) * ld + h * HD + c, xe = (size_t)(b0 + 16 * kt + r) * (ld / 32) + (h * HD + c) / 32;
         int a4[4], b4[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -1150,15 +1222,16 @@ __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __
         grava_bloco4(b4, ego - 8, (int8_t*)Gacc, (int8_t*)Ge, x + 2 * D, xe + 2 * D / 32, kid);
         return;
     }
-    soma_ondas(parc, mine, wv, lr, lg, gk);
+    int gk[ND], gvv[ND];
+    soma_ondas<HD>(parc, mine, wv, lr, lg, gk);
 #pragma unroll
-    for (int dt = 0; dt < 4; dt++)
+    for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int v = 0; v < 4; v++) mine[dt][v] = junta2(av[dt][0][v], av[dt][1][v]);
-    soma_ondas(parc, mine, wv, lr, lg, gvv);
+    soma_ondas<HD>(parc, mine, wv, lr, lg, gvv);
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const size_t o = (size_t)(b0 + jr + v) * ld + h * 64 + 16 * wv + lr;
+    for (int v = 0; v < ND; v++) {
+        const size_t o = (size_t)(b0 + jr + ND * (wv / ND) + v) * ld + h * HD + 16 * (wv % ND) + lr;
         if (gk[v] >= LIM || gk[v] <= -LIM) reporta(E_ACUM, kid, o + D, gk[v], -5);
         if (gvv[v] >= LIM || gvv[v] <= -LIM) reporta(E_ACUM, kid, o + 2 * D, gvv[v], -5);
         Gacc[o + D] = (int)gk[v];
@@ -1171,11 +1244,11 @@ __device__ __forceinline__ void atbkv_corpo(const atw::WsB& w, const uint8_t* __
 // gk, gv (workgroups [0, G)) and gq (workgroups [G, 2G)) of the backward in one launch. Both read only what
 // k_atb_prep and k_atb2 wrote and write disjoint columns of G, so their latency-bound workgroups run side by side
 // (16 KiB of LDS and at most 64 VGPRs each: all 2G workgroups of config 4 are resident at once).
-template <int NTW, int LIMITE, bool BLOCO = false>
+template <int HD, int NTW, int LIMITE, bool BLOCO = false>
 __global__ void __launch_bounds__(256) k_atbqkv(atw::WsB w, const uint8_t* __restrict__ P, int* __restrict__ Gacc, int16_t* __restrict__ Ge,
                                                 int T, int H, int D, int dsb, int kid) {
-    __shared__ __align__(16) char lds[LDS_ATBQKV<NTW>];
+    __shared__ __align__(16) char lds[LDS_ATBQKV<HD, NTW>];
     const int G = (int)gridDim.x / 2;
-    if ((int)blockIdx.x < G) atbkv_corpo<NTW, LIMITE, BLOCO>(w, P, Gacc, Ge, T, H, D, dsb, kid, lds, (int)blockIdx.x, G);
-    else atbq_corpo<NTW, LIMITE, BLOCO>(w, P, Gacc, Ge, T, H, D, dsb, kid, lds, (int)blockIdx.x - G, G);
+    if ((int)blockIdx.x < G) atbkv_corpo<HD, NTW, LIMITE, BLOCO>(w, P, Gacc, Ge, T, H, D, dsb, kid, lds, (int)blockIdx.x, G);
+    else atbq_corpo<HD, NTW, LIMITE, BLOCO>(w, P, Gacc, Ge, T, H, D, dsb, kid, lds, (int)blockIdx.x - G, G);
 }

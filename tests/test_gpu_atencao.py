@@ -68,6 +68,52 @@ def test_atencao_hd_vs_oraculo(blk, Bt, T, H, D, esp, e0, limite, via_ws):
         _cmp(a, b, nome)
 
 
+@pytest.mark.parametrize("hd,blk,Bt,T,H,esp,e0,GA,limite", [
+    (32, 32, 2, 64, 1, 3, -7, 4, False),           # one query block, one head
+    (32, 32, 1, 512, 3, 3, -7, 4, False),          # the longest rows, odd head count
+    (32, 128, 1, 320, 4, 6, -7, 4, True),          # a block spans four heads; T past 256, not a power of two
+    (32, 32, 1, 192, 2, 12, -10, 0, False),        # no guard bits, exponents far apart
+    (32, 32, 1, 128, 2, 1, 0, 4, False),           # scores shifted left
+    (16, 32, 2, 64, 2, 3, -7, 4, True),            # a block spans two heads
+    (16, 32, 1, 512, 2, 3, -7, 4, True),
+    (16, 128, 1, 448, 8, 6, -7, 2, False),
+    (16, 32, 3, 256, 6, 10, -9, 3, False),
+])
+def test_atencao_cabeca_estreita(hd, blk, Bt, T, H, esp, e0, GA, limite, monkeypatch):
+    """Head widths 32 and 16 on matrix cores (workspace) against the v_dot2 kernels of the reference ABI, bit for bit,
+    and against the oracle at the spec's GA; the backward also on a P that no forward wrote (random bytes, above the
+    diagonal too: both kernel families read the causal pairs only). Without a workspace the same entry point runs
+    the v_dot2 kernels."""
+    from jatai_amd import ops as O
+    M, D = Bt * T, hd * H
+    seed = R.substream(558, f"{hd} {blk} {T} {H} {esp} {GA} {limite}")
+    qn = R.bloco(R.substream(seed, "qkv"), M, 3 * D, blk, espalha=esp, e0=e0, zera=0.05)
+    gn = R.bloco(R.substream(seed, "go"), M, D, blk, espalha=esp, e0=-20, zera=0.05)
+    gpu = GPU(blk, vigiar=True)
+    qkv, go = (tuple(gpu.dev(v) for v in x) for x in (qn, gn))
+    Pr = gpu.dev(R.uniform_int(R.substream(seed, "P"), (Bt * H, T, T), 0, 255).astype(np.uint8))
+    monkeypatch.setattr(O, "GA", GA)
+    res = []
+    for ws in (True, False):
+        monkeypatch.setattr(O, "ATENCAO_WS", ws)
+        old = gpu.limite(limite)
+        try:
+            (oacc, oe), P = gpu.ops.atencao(qkv, Bt, T, H)
+            res.append((oacc, oe, P) + gpu.ops.atencao_back(go, qkv, P, Bt, T, H) + gpu.ops.atencao_back(go, qkv, Pr, Bt, T, H))
+        finally:
+            gpu.limite(old)
+    nomes = ("oacc", "oe", "P", "gacc", "ge", "gacc de P qualquer", "ge de P qualquer")
+    for nome, a, b in zip(nomes, *res):
+        _cmp(a, b, nome)
+    if GA == 4:
+        for nome, a, b in zip(nomes, res[0], _frente_tras(CPU(blk), qn, gn, Bt, T, H, limite)):
+            _cmp(a, b, nome + " (oracle)")
+    oacc, oe, P = (torch.zeros_like(x) for x in res[0][:3])
+    gpu.ops._lanca("atencao", "jt_atencao_ws", (*qkv, oacc, oe, P, Bt, T, H, D, GA, None, 0), dict(qkv=qkv[0], qkvE=qkv[1]), (M, D), longos=(11,))
+    for nome, a, b in zip(nomes, (oacc, oe, P), res[0]):
+        _cmp(a, b, nome + " (no workspace)")
+
+
 @pytest.mark.parametrize("T,H,limite", [(256, 8, False), (256, 8, True), (512, 4, False)])
 def test_atencao_q_igual_a_quant(T, H, limite):
     """atencao_q / atencao_back_q (outputs quantized inside the attention kernels) equal quant of the raw outputs."""
