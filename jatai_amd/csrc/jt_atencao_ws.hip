@@ -923,6 +923,9 @@ __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restr
     const int sh = atw::sh_gp_ws<LIMITE>(w, bh, T);                  // after frag_q's loads are issued
     const Desl dsh(sh);                                              // gP's shrink, one shift per head
     const uint8_t* Pb = P + (size_t)bh * T * T;
+    // bytes of the diagonal tile's rows at or past key lr. Applied by a select: a branch between a tile's MFMA and the use
+    // of its result would leave the compiler's count of the wait states in between at the longer path's
+    const unsigned causal = lr <= 4 * lg ? ~0u : lr - 4 * lg > 3 ? 0u : ~0u << (8 * (lr - 4 * lg));
     int x[NTW][4];
     unsigned pr[NTW];
     int s[4] = {0, 0, 0, 0}, pm = 0, gm = 0;
@@ -933,7 +936,7 @@ __global__ void __launch_bounds__(256) k_atb2(atw::WsB w, const uint8_t* __restr
         int o[4];
         gp_tile<HD>(w, hb, f, t, lr, lg, o);
         pr[n] = *reinterpret_cast<const unsigned*>(Pb + (size_t)j * T + i0);     // P_ij, rows i0 .. i0 + 3
-        if (HD != 64 && t == qt) pr[n] &= j <= i0 ? ~0u : j - i0 > 3 ? 0u : ~0u << (8 * (j - i0));   // causal bytes only
+        if (HD != 64) pr[n] &= t == qt ? causal : ~0u;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int xv = j <= i0 + v ? dsh(o[v]) : 0;
