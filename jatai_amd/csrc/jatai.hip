@@ -645,9 +645,12 @@ int jt_atencao(const void* qm, const void* qE, void* Oacc, void* Oe, void* P, in
     if (!alinhados(qm, qE, Oacc, Oe, P)) return (int)hipErrorInvalidValue;
     const int hd = D / H;
     if (hd == 4) {
-        if (g_linhas == 0 && T <= 128) {                 // automatic: 8 lanes per query row
-            k_atencao4l<128, 8><<<Bt * H, 1024, 0, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, (int*)Oacc, (int16_t*)Oe, (uint8_t*)P,
-                                                              T, H, D, g_blk, GA, kid);
+        if (g_linhas == 0) {                             // automatic: matrix cores, a wave per two stripes of 16 query rows
+            const size_t lds = at4::lds_frente(T);
+#define M4(TM) (lds_max(k_atencao4m<TM>, lds), k_atencao4m<TM><<<Bt * H, 2 * T, lds, g_stream>>>((const int8_t*)qm, (const int8_t*)qE, \
+               (int*)Oacc, (int16_t*)Oe, (uint8_t*)P, T, H, D, g_blk, GA, kid))
+            if (T <= 128) M4(128); else M4(256);
+#undef M4
             return fim();
         }
         const int nl = g_linhas == 2 ? 2 : 1;
@@ -749,9 +752,12 @@ int jt_atencao_back(const void* gom, const void* goE, const void* qm, const void
     const int dsb = ds_bits(T);
     if (hd == 4) {
 #define ARGS (const int8_t*)gom, (const int8_t*)goE, (const int8_t*)qm, (const int8_t*)qE, (const uint8_t*)P, (int*)Gacc, (int16_t*)Ge, T, H, D, g_blk, GA, dsb, kid
-        if (g_linhas == 0 && T <= 128) {                 // automatic: 8 lanes per query row
-            if (limite) k_atencao4l_back<128, 1, 8><<<Bt * H, 1024, 0, g_stream>>>(ARGS);
-            else k_atencao4l_back<128, 0, 8><<<Bt * H, 1024, 0, g_stream>>>(ARGS);
+        if (g_linhas == 0) {                             // automatic: matrix cores, a wave per two stripes of 16 query rows
+            const size_t lds = at4::lds_tras(T);
+#define M4(TM, LM) (lds_max(k_atencao4m_back<TM, LM>, lds), k_atencao4m_back<TM, LM><<<Bt * H, 2 * T, lds, g_stream>>>(ARGS))
+            if (T <= 128) { if (limite) M4(128, 1); else M4(128, 0); }
+            else { if (limite) M4(256, 1); else M4(256, 0); }
+#undef M4
             return fim();
         }
         const int nl = g_linhas == 2 ? 2 : 1;

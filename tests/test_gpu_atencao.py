@@ -114,6 +114,52 @@ def test_atencao_cabeca_estreita(hd, blk, Bt, T, H, esp, e0, GA, limite, monkeyp
         _cmp(a, b, nome + " (no workspace)")
 
 
+@pytest.mark.parametrize("blk,Bt,T,H,esp,e0,mmax,GA,limite", [
+    (32, 2, 32, 8, 3, -7, 127, 4, False),          # two stripes of 16 rows, the smallest
+    (128, 1, 96, 32, 3, -6, 127, 4, True),         # six: a group of four and one of two
+    (128, 2, 128, 64, 6, -6, 127, 4, False),       # the spec's shape; slopes down to 1
+    (32, 1, 128, 8, 12, -10, 127, 0, True),        # no guard bits, exponents far apart
+    (32, 1, 64, 8, 0, 0, 127, 4, False),           # a rounding shift of 1 (the integer form)
+    (128, 1, 64, 32, 1, 2, 3, 3, False),           # scores shifted left
+    (32, 1, 160, 24, 3, -7, 127, 4, True),         # past 128 keys: ten stripes
+    (128, 1, 256, 32, 3, -6, 127, 4, False),       # the longest
+    (32, 1, 256, 8, 0, -9, -128, 4, False),        # every mantissa -128: the largest sums of products (2^24)
+])
+def test_atencao4_matriz(blk, Bt, T, H, esp, e0, mmax, GA, limite, monkeypatch):
+    """Head width 4 on matrix cores (the default) against one query row per thread (jt_atencao_linhas(1)), bit for
+    bit, and against the oracle at the spec's GA; the backward also on a P that no forward wrote (random bytes, above
+    the diagonal too: both read the causal pairs only)."""
+    from jatai_amd import ops as O
+    lib = O.carrega_lib()
+    M, D = Bt * T, 4 * H
+    seed = R.substream(559, f"{blk} {T} {H} {esp} {e0} {GA} {limite}")
+    qn = R.bloco(R.substream(seed, "qkv"), M, 3 * D, blk, espalha=esp, e0=e0, zera=0.05, mmax=abs(mmax) % 128 or 127)
+    gn = R.bloco(R.substream(seed, "go"), M, D, blk, espalha=esp, e0=-20, zera=0.05)
+    if mmax < 0:
+        for m, E in (qn, gn):
+            m[:], E[:] = mmax, E.max()
+    gpu = GPU(blk, vigiar=True)
+    qkv, go = (tuple(gpu.dev(v) for v in x) for x in (qn, gn))
+    Pr = gpu.dev(R.uniform_int(R.substream(seed, "P"), (Bt * H, T, T), 0, 127).astype(np.uint8))
+    monkeypatch.setattr(O, "GA", GA)
+    res = []
+    for linhas in (0, 1):
+        lib.jt_atencao_linhas(linhas)
+        old = gpu.limite(limite)
+        try:
+            (oacc, oe), P = gpu.ops.atencao(qkv, Bt, T, H)
+            res.append((oacc, oe, P) + gpu.ops.atencao_back(go, qkv, P, Bt, T, H) + gpu.ops.atencao_back(go, qkv, Pr, Bt, T, H))
+        finally:
+            gpu.limite(old)
+            lib.jt_atencao_linhas(0)
+    nomes = ("oacc", "oe", "P", "gacc", "ge", "gacc de P qualquer", "ge de P qualquer")
+    for nome, a, b in zip(nomes, *res):
+        _cmp(a, b, nome)
+    if GA == 4:
+        for nome, a, b in zip(nomes, res[0], _frente_tras(CPU(blk), qn, gn, Bt, T, H, limite)):
+            _cmp(a, b, nome + " (oracle)")
+
+
 @pytest.mark.parametrize("T,H,limite", [(256, 8, False), (256, 8, True), (512, 4, False)])
 def test_atencao_q_igual_a_quant(T, H, limite):
     """atencao_q / atencao_back_q (outputs quantized inside the attention kernels) equal quant of the raw outputs."""
