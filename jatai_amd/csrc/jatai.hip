@@ -92,9 +92,9 @@ static void lds_max(K* k, size_t lds) {
 static bool k_ok(int K) { return K <= 4096 || (K <= 65536 && (K / g_blk) % 16 == 0); }
 
 // Tile of 32 R rows. Forced by jt_gemm_bm: 64 (R = 2) or 128 (R = 4), falling back to the tallest tile that
-// divides M (every M here is a multiple of 32). Automatic: 64 rows where that leaves at least TILES_64 tiles, 1.5 per CU
-// at BLK = 32 (each stage's B rows then serve twice the rows; us at 32 and 64 rows: 2048 x 1536, K = 512, 384 tiles,
-// 14.2 and 14.0; 2048 x 2048, K = 512, ReLU^2, 20.0 and 17.0; 4096 x 1024, K = 1024: 27.7 and 23.1; 16384 x 512, K = 2048:
+// divides M (every M here is a multiple of 32). Automatic: 64 rows where that leaves at least tiles_64() tiles, 2 per CU
+// at BLK = 32 (each stage's B rows then serve twice the rows; us at 32 and 64 rows: at 384 tiles, 2048 x 1536, K = 512,
+// 14.2 and 14.0, but the grouped weight gradients 3% slower; at 512 and more, 2048 x 2048, K = 512, ReLU^2, 20.0 and 17.0; 4096 x 1024, K = 1024: 27.7 and 23.1; 16384 x 512, K = 2048:
 // 91 and 79), 1 per CU at BLK = 128 (2048 x 1024, K = 256, ReLU^2: 7.25 and 7.05; 16384 x 1024, K = 1024: 67 and 58);
 // below that 32 rows, whose K-splits fill the chip (2048 x 512, K = 2048: 16.7 in 4 splits, 64 rows in 2: 23.0). 128 rows
 // measured within 3% of 64 where they fill the chip and slower elsewhere.
