@@ -81,3 +81,53 @@ def test_registro_estatistica_e_mensagens(tmp_path, capsys):
         assert linhas[-1]["trecho"] == "forward / mlp" and linhas[-1]["passo"] == 3
     finally:
         O.BLK = old
+
+
+def test_formato_aceita_e_recusa_sem_gpu(tmp_path):
+    """What the block-format guard accepts and refuses, over dtypes, layouts, shapes and sizes, on tensors that report
+    a GPU; one on the CPU and an operand that is no tensor are refused too."""
+    import pytest
+    import torch
+    from jatai_amd import ops as O
+    from jatai_amd.registro import ErroJatai, Registro
+
+    class NaGpu(torch.Tensor):
+        is_cuda = property(lambda self: True)
+
+    def z(*forma, tipo=torch.int8):
+        return torch.zeros(*forma, dtype=tipo).as_subclass(NaGpu)
+
+    reg, old = Registro(str(tmp_path), "f", eco=False), O.BLK
+    try:
+        for blk in (32, 128):
+            O.BLK = blk
+            for R, C in ((4, 2 * blk), (1, blk), (0, blk), (3, 0)):
+                reg.confere_bloco("A", (z(R, C), z(R, C // blk)))
+                reg.confere_r16("A", (z(R, C, tipo=torch.int16), z(R, C // blk)))
+            m, E = z(4, 2 * blk), z(4, 2)
+            for a, b, msg in ((z(4, 2 * blk, tipo=torch.int16), E, "mantissa torch.int16"), (m, z(4, 2, tipo=torch.int16), "exponent torch.int16"),
+                              (z(2 * blk, 4).t(), E, "mantissa not contiguous"), (m, z(2, 4).t(), "exponent not contiguous"),
+                              (z(4, 4 * blk)[:, ::2], E, "mantissa not contiguous"), (z(8 * blk), E, "1 dimensions"),
+                              (z(1, 4, 2 * blk), E, "3 dimensions"), (z(4, 2 * blk - 1), E, "not a multiple"), (m, z(4, 3), "exponent shape"),
+                              (m, z(2, 4), "exponent shape"), (m, z(8), "exponent shape"), (m, None, "not a tensor"), ([0], E, "not a tensor"),
+                              (torch.zeros(4, 2 * blk, dtype=torch.int8), E, "mantissa not on the GPU"),
+                              (m, torch.zeros(4, 2, dtype=torch.int8), "exponent not on the GPU")):
+                with pytest.raises(ErroJatai, match=msg):
+                    reg.confere_bloco("A", (a, b))
+    finally:
+        O.BLK = old
+
+
+def test_argumentos_c():
+    """An argument as the C call receives it: addresses (null for None and for empty tensors), ints within 32 bits,
+    and longer ones; the library's int parameters read the low 32 bits that ctypes passes."""
+    import torch
+    from jatai_amd.ops import OpsHip
+    t = torch.zeros(8, dtype=torch.int8)
+    assert OpsHip._a(t).value == t.data_ptr() and OpsHip._a(t[3:]).value == t.data_ptr() + 3
+    assert all(not OpsHip._a(x).value for x in (None, torch.empty(0), t[4:4]))
+    eco = ctypes.CDLL(None).abs                     # int abs(int): what an int parameter receives
+    for x in (0, 1, -1, 2**31 - 1, 1 - 2**31, True):
+        assert eco(OpsHip._a(x)) == abs(x)
+    for x in (2**31, -2**31, 2**40):
+        assert isinstance(OpsHip._a(x), ctypes.c_longlong) and OpsHip._a(x).value == x
