@@ -108,8 +108,7 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // values, each with its own tables (the row maxima RA, RB are over all of K). Half-size chunks keep the tables
     // of a 32-row tile at the LDS size of K = 2048, so four workgroups stay resident per CU.
     const int NBC = gemm::bloco_tab(nb, BLK, ctab);
-    // (BLK = 32: an even number of entries; the one past an odd number of blocks scales its products by 0)
-    const int nbt = BLK == 32 ? (min(nb, NBC) + 1) & ~1 : min(nb, NBC), nch = (nb + NBC - 1) / NBC;
+    const int nbt = min(nb, NBC), nch = (nb + NBC - 1) / NBC;
     // LDS: RA [BM], RB [BN] int32 (live to the end); shift terms na[b][i] = ea_ib + 4 - RA_i (int32, as termo holds it) and
     // nb[b][j] = eb_jb - RB_j (int8) of the chunk's blocks, clamped at -100 (n = na + nb <= -22 scales |p| < 2^21
     // below 1/2, i.e. to 0, as rnd(., s >= 26) does); then the stage buffers [KS][2][STAGE], which first hold the
@@ -132,7 +131,7 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     // Stage loads through buffer resources of the tile's A rows and B rows (bounds: the tile's own bytes, so no
     // access leaves them): the stage offset is the scalar operand, the lane offsets stay fixed, and a stage takes no
     // vector address arithmetic. The last stage may extend past K (nb not a multiple of the blocks per stage): its
-    // vectors past K re-read the row's last vector instead (those bytes land in a block past nb, skipped or scaled by 0).
+    // vectors past K re-read the row's last vector instead (those bytes land in a block past nb, never computed).
     const auto rsA = __builtin_amdgcn_make_buffer_rsrc((void*)(A + (size_t)row0 * K), (short)0, BM * K, 0x00020000);
     const auto rsB = __builtin_amdgcn_make_buffer_rsrc((void*)(B + (size_t)col0 * K), (short)0, BN * K, 0x00020000);
     int voff[NL];
@@ -277,10 +276,6 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
             else rb_s[tid - OB] = m;
         }
         __syncthreads();
-        if (nbt > nb) {
-            if (tid < BM) na_s[nb * BM + tid] = 0;
-            if (tid < BN) nb_s[nb * BN + tid] = 0;
-        }
         desloca_tab(nb, sst1);
     };
     // one chunk whose exponent rows are whole 16-byte vectors, at most 8 per row (K <= 4096): no staging. A row is
@@ -426,10 +421,10 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
             produtos(tile, 0, p);
             arredonda(st * 2, p);
             int f = 0;                                              // bit 23 of a sum's bits: it left [2^23, 2^24)
-            // the second block of an odd number's last stage has scales of 0 and adds nothing; 32-row tiles, whose
-            // threads hold more stage rows, still skip it: without the branch both blocks' addresses stay live in
-            // registers and spill (M = 16384, N = 1536, K = 512 at 32 rows: 76 us with it, 99 without)
-            if (R > 1 || st * 2 + 1 < nb) {
+            // an odd number's last stage has no second block. The branch pays at every number of blocks: without it both
+            // blocks' addresses stay live in registers (M = 16384, N = 2048: 43.5 -> 40.5 us at K = 32, 98 -> 93 at 512, 299
+            // -> 286 at 2048, 64-row tiles; at 32 rows they spill: N = 1536, K = 512, 76 us with it, 99 without)
+            if (st * 2 + 1 < nb) {
                 v4i q[2][2];
                 produtos(tile, 1, q);
                 arredonda(st * 2 + 1, q);
@@ -779,8 +774,7 @@ static inline size_t gemm_lds(int nb, int ks, int blk, int R = 1, int ctab = 0) 
     using gemm::PAD;
     const int bm = 32 * R;
     nb = std::min(nb, gemm::bloco_tab(nb, blk, ctab));              // the shift tables hold one chunk of K
-    const size_t nbt = blk == 32 ? (nb + 1) & ~1 : nb;
-    const size_t fixo = (size_t)(bm + BN) * 4 + nbt * bm * 4 + ((nbt * BN + 15) & ~(size_t)15);
+    const size_t fixo = (size_t)(bm + BN) * 4 + (size_t)nb * bm * 4 + (((size_t)nb * BN + 15) & ~(size_t)15);
     const size_t stage = (size_t)(32 * R + BN) * (blk == 32 ? gemm::Est<32>::LD : gemm::Est<128>::LD);
     size_t area = (size_t)ks * 2 * stage;
     const size_t exp_bruto = (size_t)(nb + 4) * (bm + BN + 1) + 16;   // staged rows nb + 4 bytes apart, and a junk row

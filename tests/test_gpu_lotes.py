@@ -176,3 +176,23 @@ def test_gemm_arredondamento_fp32(M, N, K, bm):
         ref = cpu.ops.gemm(*[tuple(torch.from_numpy(v) for v in x) for x in t], cru=True)
         for a, b in zip(out, ref):
             assert np.array_equal(host(a), host(b)), f"{M}x{N}x{K} case {caso}"
+
+
+@pytest.mark.parametrize("K", [32, 96, 288, 544, 2080, 4064])
+@pytest.mark.parametrize("bm", [32, 64, 128])
+def test_gemm_numero_impar_de_blocos(K, bm):
+    """An odd number of 32-value blocks of K (the last stage holds one, not two) at every tile height, raw and in the
+    grouped launch, against the oracle: the bytes past K in that stage take no part, whatever they are."""
+    M, N, blk = 128, 128, 32
+    gpu, cpu = GPU(blk, vigiar=True), CPU(blk)
+    A, B = (R.bloco(R.substream(137, f"{K} {n}"), L, K, blk, espalha=3, e0=-8, zera=0.05) for n, L in (("A", M), ("B", N)))
+    ref = cpu.ops.gemm(*[tuple(torch.from_numpy(v) for v in x) for x in (A, B)], cru=True)
+    A, B = (tuple(gpu.dev(v) for v in x) for x in (A, B))
+    gpu.ops.lib.jt_gemm_bm(bm)
+    try:
+        outs = [gpu.ops.gemm(A, B, cru=True), *gpu.ops.gemm_cru_lote([(A, B, None), (A, B, None)])]
+    finally:
+        gpu.ops.lib.jt_gemm_bm(0)
+    for out in outs:
+        for a, b in zip(out, ref):
+            assert np.array_equal(host(a), host(b)), (K, bm)
