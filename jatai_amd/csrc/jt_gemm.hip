@@ -512,12 +512,17 @@ __device__ __forceinline__ void gemm_corpo(const int8_t* __restrict__ A, const i
     }
     int* acc_s = reinterpret_cast<int*>(buf);                      // [KS][BM][BN + PAD]
     constexpr int TILE = BM * (BN + PAD);
+    // mode 4 at 32 rows computes the lane's place in the tile again, from an opaque copy of the lane: kept in a register
+    // from before the K loop it was spilled around the loop (16 bytes of scratch per thread; the time is the same)
+    int le = lane;
+    if constexpr (MODO == 4 && R == 1) asm("" : "+v"(le));
+    const int lre = le & 15, lge = le >> 4;
 #pragma unroll
     for (int ti = 0; ti < 2; ti++)
 #pragma unroll
         for (int tj = 0; tj < 2; tj++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc_s[g * TILE + (wr + 16 * ti + 4 * lg + i) * (BN + PAD) + wc + 16 * tj + lr] = acc[ti][tj][i];
+            for (int i = 0; i < 4; i++) acc_s[g * TILE + (wr + 16 * ti + 4 * lge + i) * (BN + PAD) + wc + 16 * tj + lre] = acc[ti][tj][i];
     if (fora) {                                                     // K > 4096 only: an accumulator out of range
         const int e = __builtin_ctz(fora), ti = e >> 3, tj = (e >> 2) & 1, i = e & 3;
         reporta(E_ACUM, kid, (long long)(row0 + wr + 16 * ti + 4 * lg + i) * N + col0 + wc + 16 * tj + lr,
