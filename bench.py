@@ -127,7 +127,7 @@ def gemm_formas(c):
 def gemm_kernel(O, ops, M, N, K, modo):
     """Symbol and grid the library launches for this shape, to match rocprof rows."""
     ks = ops.lib.jt_gemm_divisoes(M, N, K, modo)
-    bm = ops.lib.jt_gemm_tile(M, N, modo)
+    bm = ops.lib.jt_gemm_tile_k(M, N, K, modo)
     return {"symbol": f"k_gemm<{O.BLK}, {modo}, {ks}, {bm // 32}>", "workgroups": (M // bm) * (N // 128),
             "threads": 256 * (bm // 32) * ks, "tile_rows": bm}
 
@@ -213,12 +213,11 @@ def mede_dw_lote(O, ops, c, rep=7):
     del grafo
     ms = sorted(vezes)[len(vezes) // 2]
     ops_alg = sum(2 * M * N * K for _, M, N in formas)
-    r = 2 if all(M % 64 == 0 for _, M, _ in formas) and sum((M // 64) * (N // 128) for _, M, N in formas) >= (512 if blk == 32 else 256) else 1
-    tiles = sum((M // (32 * r)) * (N // 128) for _, M, N in formas)
+    # the group takes the tile and the splits of one raw product with as many tiles (every M here is a multiple of 128)
     lote = 64                                   # GEMMs per grouped launch (LOTE_G)
-    nk = 1
-    while nk < 4 // r and tiles * r * 2 * nk <= 1024 and (K // blk) >= 8 * nk:
-        nk *= 2
+    t32 = sum((M // 32) * (N // 128) for _, M, N in formas[:lote])
+    r, nk = ops.lib.jt_gemm_tile_k(32 * t32, 128, K, 1) // 32, ops.lib.jt_gemm_divisoes(32 * t32, 128, K, 1)
+    tiles = sum((M // (32 * r)) * (N // 128) for _, M, N in formas)
     return dict(ms=ms, ms_each=[round(x, 4) for x in vezes], ops=ops_alg, gemms=len(formas), K=K, launches=(len(formas) + lote - 1) // lote,
                 symbol=f"k_gemm_lote<{blk}, {nk}, {r}>", workgroups=tiles, threads=256 * r * nk)
 

@@ -51,8 +51,9 @@ int jt_gemm_f(const void* A, const void* EA, const void* B, const void* EB, void
               const void* Xm, const void* XE, void* Om2, void* OE2, int M, int N, int K, int modo, int kid);
 int jt_gemm_divisoes(int M, int N, int K, int modo);   /* no reference counterpart: K-splits jt_gemm_f uses
                                                         * for a shape (workgroup = 256 x tile rows / 32 x splits threads) */
-int jt_gemm_tile(int M, int N, int modo);              /* no reference counterpart: tile rows (32, 64, 128) jt_gemm_f
-                                                        * uses for a shape and mode */
+int jt_gemm_tile_k(int M, int N, int K, int modo);     /* no reference counterpart: tile rows (32, 64, 128) jt_gemm_f
+                                                        * uses for a shape and mode; jt_gemm_tile: for K = 512 to 3936 */
+int jt_gemm_tile(int M, int N, int modo);
 int jt_gemm(const void* A, const void* EA, const void* B, const void* EB, void* Cm, void* CE, void* C32, void* Ce,
             int M, int N, int K, int modo, int kid);
 /* no reference counterpart: Z16 = soma16(X16, A.B^T) (R16, int16 mantissas) and Y8 = para8(Z16) in one launch, the

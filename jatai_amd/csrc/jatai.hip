@@ -92,16 +92,42 @@ static void lds_max(K* k, size_t lds) {
 static bool k_ok(int K) { return K <= 4096 || (K <= 65536 && (K / g_blk) % 16 == 0); }
 
 // Tile of 32 R rows. Forced by jt_gemm_bm: 64 (R = 2) or 128 (R = 4), falling back to the tallest tile that
-// divides M (every M here is a multiple of 32). Automatic: 64 rows where that leaves at least tiles_64() tiles, 2 per CU
-// at BLK = 32 (each stage's B rows then serve twice the rows; us at 32 and 64 rows: at 384 tiles, 2048 x 1536, K = 512,
-// 14.2 and 14.0, but the grouped weight gradients 3% slower; at 512 and more, 2048 x 2048, K = 512, ReLU^2, 20.0 and 17.0; 4096 x 1024, K = 1024: 27.7 and 23.1; 16384 x 512, K = 2048:
-// 91 and 79), 1 per CU at BLK = 128 (2048 x 1024, K = 256, ReLU^2: 7.25 and 7.05; 16384 x 1024, K = 1024: 67 and 58);
-// below that 32 rows, whose K-splits fill the chip (2048 x 512, K = 2048: 16.7 in 4 splits, 64 rows in 2: 23.0). 128 rows
-// measured within 3% of 64 where they fill the chip and slower elsewhere.
-static long long tiles_64() { return g_blk == 32 ? 512 : 256; }
-static int gemm_r(int M, int N) {
+// divides M (every M here is a multiple of 32). Automatic: 64 rows, whose stages of B serve twice the rows, where all of
+// these hold, else 32 (us at 32 and at 64 rows, launches back to back in a graph, block outputs unless said otherwise):
+// - the 64-row tiles number one per CU or more (2048 x 1024: K = 512 10.8 and 10.1; BLK 128, K = 1024 16.8 and 11.9). With
+//   fewer, 32-row tiles and their K-splits fill the chip (2048 x 512, K = 2048: 16.4 and 23.0).
+// - they give no CU more rows than 32-row tiles do: twice their number per CU, rounded up, is at most that of 32-row tiles.
+//   BLK 32, K = 512: 13.3 and 14.3 with 384 of them (1.5 per CU), 15.8 and 14.7 with 448, 20.4 and 21.2 with 640, 23.2 and
+//   21.9 with 768; BLK 128, K = 256: 8.1 and 8.6 with 384, 10.9 and 8.9 with 448. Past 4 per CU the uneven rest weighs little
+//   (1152, K = 1024: 53.0 and 53.5; a group of 2160, K = 2048: 184 and 183), at BLK 128, where 3 of the 32-row workgroups
+//   fit a CU, already past 3 (896, K = 256: 16.6 and 15.4), and past 2 from K = 512 on (640, K = 1024, mode 4: 27.6 and 26.8).
+// - K outweighs the prologue and the epilogue, which more, smaller tiles overlap better (BLK 32): K >= 64 (4096 x 1024: K =
+//   32 6.9 and 7.1, K = 64 7.3 and 7.2); with more than 4 tiles per CU K >= 512 (16384 x 2048: K = 256 66.2 and 67.7, K = 512
+//   94.0 and 91.4); for raw outputs, whose epilogue writes 6 bytes a value, too (8192 x 1024: K = 64 13.7 and 14.8, K = 512
+//   30.2 and 29.2; a group of 1152: K = 128 21.0 and 22.3, K = 3072 152 and 144). At BLK 128 only for raw outputs whose
+//   32-row tiles fit in one round (2048 x 1024, K = 128 6.8 and 7.2; 4096 x 1024 10.7 and 9.2).
+// - two such workgroups fit a CU's LDS, which the shift tables of K > 3936 in one chunk do not leave at BLK 32 (8192 x 2048,
+//   K = 4096: 416 and 407). 128-row tiles, 16 waves in one workgroup, take 306 there and are chosen where they give every CU
+//   one and no CU over 4/3 of the rows that 32-row tiles do (a group of 1152 64-row tiles, 12 against 9:
+//   240 and 223; 640, 8 against 5, would leave most CUs idle in a second round).
+// 128 rows also for modes 3 and 4 at BLK 128 where they make one tile per CU (4096 x 1024, mode 4: K = 768 16.0 at 64 rows,
+// 15.6; K = 3072 38.0, 36.6; mode 3, whose epilogue is heavier, from K = 1024 on: K = 3072 37.5, 36.7). Elsewhere 128 rows are
+// within 3% of 64 where they fill the chip evenly and slower otherwise.
+static int gemm_r_auto(long long t64, bool m128, int K, int modo) {    // t64: the product's or group's 64-row tiles, 0 if M % 64
+    const long long cu = 256;
+    auto carga = [&](long long tiles, int linhas) { return linhas * ((tiles + cu - 1) / cu); };   // of the fullest CU, in 32 rows
+    const long long c32 = carga(2 * t64, 1);
+    if (t64 < cu) return 1;
+    if (2 * gemm_lds(K / g_blk, 1, g_blk, 2) > 160 * 1024) return t64 >= 2 * cu && m128 && 3 * carga(t64 / 2, 4) <= 4 * c32 ? 4 : 1;
+    if (carga(t64, 2) > c32 && t64 <= (g_blk == 32 ? 4 * cu : K < 512 ? 3 * cu : 2 * cu)) return 1;
+    if (g_blk == 32 && (K < 64 || (K < 512 && (modo == 1 || t64 > 4 * cu)))) return 1;
+    if (g_blk == 128 && modo == 1 && K < 512 && 2 * t64 <= 3 * cu) return 1;
+    if (g_blk == 128 && (modo == 4 || (modo == 3 && K >= 1024)) && t64 == 2 * cu && m128) return 4;
+    return 2;
+}
+static int gemm_r(int M, int N, int K, int modo) {
+    if (g_gemm_bm == 0) return gemm_r_auto(M % 64 ? 0 : (long long)(M / 64) * (N / 128), M % 128 == 0, K, modo);
     int r = g_gemm_bm >= 128 ? 4 : g_gemm_bm >= 64 ? 2 : 1;
-    if (g_gemm_bm == 0 && M % 64 == 0 && (long long)(M / 64) * (N / 128) >= tiles_64()) r = 2;
     while (r > 1 && M % (32 * r)) r /= 2;
     return r;
 }
@@ -112,7 +138,7 @@ static int gemm_divisoes_r(int M, int N, int K, int modo, int r) {
     while (ks < ksmax && tiles * r * 2 * ks <= g_alvo_wg && nb >= 8 * ks) ks *= 2;
     return ks;
 }
-static int gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes_r(M, N, K, modo, gemm_r(M, N)); }
+static int gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes_r(M, N, K, modo, gemm_r(M, N, K, modo)); }
 
 extern "C" {
 
@@ -180,8 +206,10 @@ int jt_bloco_atual() { return g_blk; }
 // ---------------------------------------------------------------------------------------------- GEMM
 // No reference counterpart: the K-split count jt_gemm_f uses for a shape (workgroup = 256 x splits threads).
 int jt_gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes(M, N, K, modo); }
-// No reference counterpart: the tile rows (32, 64 or 128) jt_gemm_f uses for a shape and mode.
-int jt_gemm_tile(int M, int N, int modo) { (void)modo; return 32 * gemm_r(M, N); }
+// No reference counterpart: the tile rows (32, 64 or 128) jt_gemm_f uses for a shape and mode; jt_gemm_tile is for the K
+// between 512 and 3936, where the rows do not depend on it.
+int jt_gemm_tile_k(int M, int N, int K, int modo) { return 32 * gemm_r(M, N, K, modo); }
+int jt_gemm_tile(int M, int N, int modo) { return 32 * gemm_r(M, N, 512, modo); }
 }  // extern "C"
 // modes 0-4 (jt_gemm_f) and 6 (jt_gemm_soma16)
 static int gemm_f(const void* A, const void* EA, const void* B, const void* EB, void* Cm, void* CE, void* C32, void* Ce, const void* Xm,
@@ -189,7 +217,7 @@ static int gemm_f(const void* A, const void* EA, const void* B, const void* EB, 
     using namespace gemm;
     if (M <= 0 || N <= 0 || K <= 0 || M % BM || N % BN || K % g_blk || !k_ok(K)) return (int)hipErrorInvalidValue;
     if (!alinhados(A, EA, B, EB, Cm, CE, C32, Ce, Xm, XE, Om2, OE2)) return (int)hipErrorInvalidValue;
-    const int nb = K / g_blk, r = gemm_r(M, N);
+    const int nb = K / g_blk, r = gemm_r(M, N, K, modo);
     // mode 4 with Om2 (T(gh)) and mode 3 with C32, Ce (T(a)): the transposed copy needs a single K-split (BLK = 32 only)
     if (modo == 4 && (Om2 || OE2) && (g_blk != 32 || !Om2 || !OE2)) return (int)hipErrorInvalidValue;
     if (modo == 3 && (C32 || Ce) && (g_blk != 32 || !C32 || !Ce)) return (int)hipErrorInvalidValue;
@@ -254,15 +282,18 @@ int jt_gemm_lote(const void* entradas, int n, int kid) {
         L.n = std::min(LOTE_G, n - base);
         L.K = e[base].K;
         L.compacto = e[base].compacto;
-        // the tallest forced tile every M of the group allows, or 64 rows by the rule of gemm_r with the group's tiles
-        int r = g_gemm_bm == 0 ? 2 : 4;
+        // the tallest forced tile every M of the group allows, or by the rule of one raw product with the group's tiles
+        int r = 4;
         long long t64 = 0;
+        bool m64 = true, m128 = true;
         for (int i = 0; i < L.n; i++) {
             const int Mi = e[base + i].M > 0 ? e[base + i].M : 32;
-            r = std::min(r, g_gemm_bm == 0 ? (Mi % 64 == 0 ? 2 : 1) : gemm_r(Mi, 0));
+            if (g_gemm_bm != 0) r = std::min(r, gemm_r(Mi, 0, L.K, 1));
+            m64 = m64 && Mi % 64 == 0;
+            m128 = m128 && Mi % 128 == 0;
             t64 += (long long)(Mi / 64) * (std::max(e[base + i].N, 0) / BN);
         }
-        if (g_gemm_bm == 0 && t64 < tiles_64()) r = 1;
+        if (g_gemm_bm == 0) r = gemm_r_auto(m64 ? t64 : 0, m128, L.K, 1);
         long long tot = 0;
         for (int i = 0; i < L.n; i++) {
             const EntradaG& x = e[base + i];

@@ -153,3 +153,33 @@ def test_kernels_sem_scratch(tmp_path):
     scratch, derramados = campos("private_segment_fixed_size"), campos("vgpr_spill_count")
     assert len(nomes) == len(scratch) == len(derramados) > 100
     assert not [x for x in zip(nomes, scratch, derramados) if x[1:] != ("0", "0")]
+
+
+def test_linhas_do_tile_sem_gpu():
+    """The GEMM's automatic tile on both sides of each line of its rule: tiles per CU, an uneven load, short K, raw
+    outputs, the LDS of a long K, and an M that a taller tile does not divide; forced tiles ignore the rule."""
+    from jatai_amd.ops import carrega_lib
+    lib = carrega_lib()
+    antes = lib.jt_bloco_atual()
+    try:
+        for blk, M, N, K, modo, linhas in (
+                (32, 1984, 1024, 512, 0, 32), (32, 2048, 1024, 512, 0, 64),                                    # one 64-row tile per CU
+                (32, 2048, 1536, 512, 0, 32), (32, 3584, 1024, 512, 0, 64), (32, 5120, 1024, 512, 0, 32),      # even and uneven loads
+                (128, 2048, 1536, 256, 0, 32), (128, 3584, 1024, 256, 0, 64), (32, 9216, 1024, 512, 0, 64),
+                (32, 2048, 2048, 32, 0, 32), (32, 2048, 2048, 64, 0, 64), (32, 2048, 2048, 480, 1, 32), (32, 2048, 2048, 512, 1, 64),
+                (32, 16384, 2048, 480, 0, 32), (32, 16384, 2048, 512, 0, 64), (128, 2048, 1024, 128, 1, 32), (128, 4096, 1024, 128, 1, 64),
+                (32, 2048, 2048, 3936, 4, 64), (32, 2048, 2048, 3968, 4, 128), (32, 2048, 2048, 4096, 0, 128), (32, 2048, 1024, 4096, 0, 32),
+                (32, 8256, 1024, 4096, 0, 32), (32, 5120, 1024, 4096, 0, 32), (32, 7168, 1024, 4096, 3, 128), (32, 2048, 2048, 8192, 0, 64),
+                (128, 2048, 2048, 256, 4, 128), (128, 2048, 2048, 896, 3, 64), (128, 2048, 2048, 1024, 3, 128),
+                (128, 5120, 1024, 384, 0, 32), (128, 7168, 1024, 384, 0, 64), (128, 5120, 1024, 512, 0, 64), (32, 4128, 1024, 512, 0, 32)):
+            lib.jt_bloco(blk)
+            assert lib.jt_gemm_tile_k(M, N, K, modo) == linhas, (blk, M, N, K, modo)
+            if K == 512:
+                assert lib.jt_gemm_tile(M, N, modo) == linhas
+            for bm in (32, 64, 128):
+                lib.jt_gemm_bm(bm)
+                assert lib.jt_gemm_tile_k(M, N, K, modo) == max(r for r in (32, 64, 128) if r <= bm and M % r == 0)
+            lib.jt_gemm_bm(0)
+    finally:
+        lib.jt_gemm_bm(0)
+        lib.jt_bloco(antes)

@@ -196,3 +196,30 @@ def test_gemm_numero_impar_de_blocos(K, bm):
     for out in outs:
         for a, b in zip(out, ref):
             assert np.array_equal(host(a), host(b)), (K, bm)
+
+
+@pytest.mark.parametrize("blk,M,N,K,bm", [(32, 2048, 1024, 64, 64), (32, 3584, 1024, 544, 64), (32, 2048, 2048, 3936, 64), (32, 2048, 2048, 3968, 128),
+                                          (32, 2048, 2048, 4096, 128), (32, 8256, 1024, 4096, 32), (32, 2048, 2048, 32, 32),
+                                          (128, 2048, 2048, 128, 128), (128, 3584, 1024, 1152, 64), (128, 2048, 1536, 256, 32)])
+def test_gemm_tile_automatico(blk, M, N, K, bm):
+    """Every fused form and the grouped launch with the tile the rule takes for the shape, against 32-row tiles (held to
+    the oracle at small shapes): the same bits. bm: the ReLU^2-backward product's tile."""
+    gpu = GPU(blk, vigiar=True)
+    assert gpu.ops.lib.jt_bloco(blk) == 0 and gpu.ops.lib.jt_gemm_tile_k(M, N, K, 4) == bm
+    s = lambda n: R.substream(139, f"{blk} {M} {N} {K} {n}")
+    A, B, X = (tuple(gpu.dev(v) for v in R.bloco(s(n), L, C, blk, espalha=3, e0=-8)) for n, L, C in (("A", M, K), ("B", N, K), ("X", M, N)))
+
+    def formas():
+        o = gpu.ops
+        sai = [o.gemm(A, B), o.gemm(A, B, cru=True), o.gemm_soma(A, B, X), *o.gemm_relu2(A, B), o.gemm_relu2_back(A, B, X),
+               *o.gemm_cru_lote([(A, B, None), (A, B, None)])]
+        if blk == 32 and M % 128 == 0:
+            sai += [*o.gemm_relu2_t(A, B), *o.gemm_relu2_back_t(A, B, X)]
+        return [t for x in sai for t in x]
+    auto = formas()
+    gpu.ops.lib.jt_gemm_bm(32)
+    try:
+        ref = formas()
+    finally:
+        gpu.ops.lib.jt_gemm_bm(0)
+    assert len(auto) == len(ref) and all(torch.equal(a, b) for a, b in zip(auto, ref))
