@@ -277,8 +277,10 @@ __device__ __forceinline__ int grupo_max(int v, int (&red)[8], int n) {
     __syncthreads();
     return max(max(max(red[0], red[1]), max(red[2], red[3])), max(max(red[4], red[5]), max(red[6], red[7])));
 }
-// Eight wait states after the last MFMA of an accumulator whose use follows a branch: the compiler counts the states
-// between an MFMA and a use of its result along one path only, and a use reached by two paths can read too early
+// Eight wait states after the last MFMA of an accumulator whose use more than one path reaches: the compiler counts the
+// states between an MFMA and a use of its result along one path only, and can leave too few on another. A use that a single
+// path reaches (gv's drain below, behind a branch of its own) has the compiler's own wait. tests/test_codigo.py counts the
+// states of every MFMA of the built library on every path.
 __device__ __forceinline__ void pronto(f4_t& a) { asm volatile("s_nop 7" : "+v"(a)); }
 // pieces of four dS: d = a 2^LB + b
 template <int LB>

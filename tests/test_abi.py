@@ -133,28 +133,6 @@ def test_argumentos_c():
         assert isinstance(OpsHip._a(x), ctypes.c_longlong) and OpsHip._a(x).value == x
 
 
-def test_kernels_sem_scratch(tmp_path):
-    """No kernel of the built library keeps registers in scratch memory: the code object's own metadata."""
-    import shutil
-    import subprocess
-
-    import pytest
-    from jatai_amd.build import HIPCC
-    from jatai_amd.ops import LIB
-    llvm = os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "llvm", "bin")
-    if not os.path.exists(os.path.join(llvm, "llvm-readelf")):
-        pytest.skip("no llvm-readelf beside hipcc")
-    so = shutil.copy(LIB, tmp_path)
-    subprocess.run([os.path.join(llvm, "llvm-objdump"), "--offloading", so], check=True, capture_output=True, cwd=tmp_path)
-    co, = tmp_path.glob("*gfx950*")
-    notas = subprocess.run([os.path.join(llvm, "llvm-readelf"), "--notes", co], check=True, capture_output=True, text=True).stdout
-    campos = lambda c: re.findall(rf"^\s*-?\s*\.{c}:\s+(\S+)", notas, re.M)
-    nomes = [n for n in campos("symbol") if n.endswith(".kd")]
-    scratch, derramados = campos("private_segment_fixed_size"), campos("vgpr_spill_count")
-    assert len(nomes) == len(scratch) == len(derramados) > 100
-    assert not [x for x in zip(nomes, scratch, derramados) if x[1:] != ("0", "0")]
-
-
 def test_linhas_do_tile_sem_gpu():
     """The GEMM's automatic tile on both sides of each line of its rule: tiles per CU, an uneven load, short K, raw
     outputs, the LDS of a long K, and an M that a taller tile does not divide; forced tiles ignore the rule."""
