@@ -127,8 +127,9 @@ def test_atencao_cabeca_estreita(hd, blk, Bt, T, H, esp, e0, GA, limite, monkeyp
 ])
 def test_atencao4_matriz(blk, Bt, T, H, esp, e0, mmax, GA, limite, monkeypatch):
     """Head width 4 on matrix cores (the default) against one query row per thread (jt_atencao_linhas(1)), bit for
-    bit, and against the oracle at the spec's GA; the backward also on a P that no forward wrote (random bytes, above
-    the diagonal too: both read the causal pairs only)."""
+    bit, and against the oracle at the spec's GA; the backward also on a P that no forward wrote (random values of 0 to
+    127, above the diagonal too: both read the causal pairs only; a row sum of P gP' stays below 2^30 at T = 256 only for
+    such P. test_atencao4_p_denso has the larger ones)."""
     from jatai_amd import ops as O
     lib = O.carrega_lib()
     M, D = Bt * T, 4 * H
@@ -158,6 +159,47 @@ def test_atencao4_matriz(blk, Bt, T, H, esp, e0, mmax, GA, limite, monkeypatch):
     if GA == 4:
         for nome, a, b in zip(nomes, res[0], _frente_tras(CPU(blk), qn, gn, Bt, T, H, limite)):
             _cmp(a, b, nome + " (oracle)")
+
+
+@pytest.mark.parametrize("blk,Bt,T,H,cheio,vmax,limite", [
+    (32, 2, 32, 8, False, 127, False),             # every byte value; |sum P gP'| <= 255 2^15 T < 2^30 up to T = 128
+    (128, 1, 96, 32, False, 127, True),
+    (32, 1, 128, 8, False, 127, False),
+    (32, 1, 64, 8, True, 1, False),                # P = 255 and |dO| = 2048: two tiles' sum of gv is 32 255 2048 = 0.996 2^24
+    (32, 1, 96, 8, True, 1, True),
+    (128, 1, 128, 32, True, 1, False),             # |gP| = 4 2048 16 -> |gP'| = 2^14
+    (32, 1, 256, 8, True, 0, False),               # the longest column; v = 0 keeps the row sums at 0
+])
+def test_atencao4_p_denso(blk, Bt, T, H, cheio, vmax, limite):
+    """The backward at head width 4 on matrix cores with P over all of 0 .. 255, or 255 in every causal pair with every
+    |dO| at its largest (mantissas of -128, one exponent), where the unpacking of P's top bit and gv's exact fp32 sums are
+    at their edges: one query row per thread (jt_atencao_linhas(1)) and the oracle give the same bits."""
+    from jatai_amd import ops as O
+    lib = O.carrega_lib()
+    M, D = Bt * T, 4 * H
+    seed = R.substream(560, f"{blk} {T} {H} {cheio} {limite}")
+    qn = R.bloco(R.substream(seed, "qkv"), M, 3 * D, blk, espalha=3, e0=-7)
+    gn = R.bloco(R.substream(seed, "go"), M, D, blk, espalha=3, e0=-20)
+    P = R.uniform_int(R.substream(seed, "P"), (Bt * H, T, T), 0, 255).astype(np.uint8)
+    if cheio:
+        P[:] = 255
+        gn[0][:], gn[1][:] = -128, -20
+        qn[0][:, 2 * D:] = np.clip(qn[0][:, 2 * D:], -vmax, vmax)
+        qn[1][:, 2 * D // blk:] = -7
+    P *= (np.arange(T)[None, :] >= np.arange(T)[:, None]).astype(np.uint8)       # P[j, i], keys j up to the query i
+    gpu, cpu = GPU(blk, vigiar=True), CPU(blk)
+    res = []
+    for be, linhas in ((gpu, 0), (gpu, 1), (cpu, 0)):
+        lib.jt_atencao_linhas(linhas)
+        old = be.limite(limite)
+        try:
+            res.append(be.ops.atencao_back(tuple(be.dev(v) for v in gn), tuple(be.dev(v) for v in qn), be.dev(P), Bt, T, H))
+        finally:
+            be.limite(old)
+            lib.jt_atencao_linhas(0)
+    for nome, a, b, c in zip(("gacc", "ge"), *res):
+        _cmp(a, b, nome)
+        _cmp(a, c, nome + " (oracle)")
 
 
 @pytest.mark.parametrize("T,H,limite", [(256, 8, False), (256, 8, True), (512, 4, False)])
