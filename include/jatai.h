@@ -26,8 +26,8 @@ void jt_stream(void* stream);          /* every later launch goes to this hipStr
 
 /* ---- tuning knobs (jatai_cuda.cu:1087-1091) */
 void jt_gemm_split(int alvo_wg);       /* split-K target workgroup count for raw GEMM outputs */
-void jt_gemm_bm(int bm);               /* jatai_cuda.cu:1090: GEMM tile rows: 0 automatic (64 on large grids, else 32; 32 too),
-                                        * 64 or 128 forced; a forced tile that does not divide M falls back to one that does; same bits */
+void jt_gemm_bm(int bm);               /* jatai_cuda.cu:1090: GEMM tile rows: 0 automatic (32, 64 or 128 by the shape), or 32,
+                                        * 64, 128 forced; a forced tile that does not divide M falls back to one that does; same bits */
 void jt_atencao_linhas(int n);         /* jatai_cuda.cu:1091: query rows per thread of the head-width-4 attention: 1 or 2 (rows
                                         * i and T - 1 - i); any other value (0, the default) is automatic: matrix cores, a wave
                                         * per two stripes of 16 query rows; same bits */

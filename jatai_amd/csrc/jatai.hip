@@ -182,12 +182,13 @@ int jt_erro_limpa() {
 int jt_sincroniza() { return (int)hipDeviceSynchronize(); }
 void jt_stream(void* st) { g_stream = (hipStream_t)st; }
 void jt_gemm_split(int alvo) { g_alvo_wg = alvo > 0 ? alvo : 1024; }
-// jatai_cuda.cu:1090: GEMM tile rows, 0 automatic (32), or 64 / 128 forced (32 forces the default); same bits.
+// jatai_cuda.cu:1090: GEMM tile rows, 0 automatic (gemm_r_auto), or 32, 64, 128 forced; same bits.
 void jt_gemm_bm(int bm) { g_gemm_bm = bm; }
-// jatai_cuda.cu:1091: query rows per thread of the head-width-4 attention, 1 (default) or 2 (rows i and T - 1 - i,
-// which balances the causal work); same bits.
+// jatai_cuda.cu:1091: query rows per thread of the head-width-4 attention, 1 or 2 (rows i and T - 1 - i, which balances
+// the causal work); any other value (0, the default) is automatic: matrix cores. Same bits.
 void jt_atencao_linhas(int n) { g_linhas = n == 1 || n == 2 ? n : 0; }
-// No reference counterpart: selects the matrix-core (1, default) or dot2 (0) attention kernels at head width 64.
+// No reference counterpart: selects the matrix-core (1, default) or dot2 (0) attention kernels at head widths 64, 32 and
+// 16 (32 and 16: with a workspace).
 void jt_atencao_mfma(int ligado) { g_atencao_mfma = ligado ? 1 : 0; }
 // jatai_cuda.cu:1087: stochastic rounding of gemm_soma's residual add. A synchronous copy into the device global
 // g_res_est of the current device; gemm_soma kernels read it when they run.
@@ -204,7 +205,7 @@ int jt_bloco(int blk) {
 int jt_bloco_atual() { return g_blk; }
 
 // ---------------------------------------------------------------------------------------------- GEMM
-// No reference counterpart: the K-split count jt_gemm_f uses for a shape (workgroup = 256 x splits threads).
+// No reference counterpart: the K-split count jt_gemm_f uses for a shape (workgroup = 256 x tile rows / 32 x splits threads).
 int jt_gemm_divisoes(int M, int N, int K, int modo) { return gemm_divisoes(M, N, K, modo); }
 // No reference counterpart: the tile rows (32, 64 or 128) jt_gemm_f uses for a shape and mode; jt_gemm_tile is for the K
 // between 512 and 3936, where the rows do not depend on it.

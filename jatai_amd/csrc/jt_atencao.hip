@@ -248,7 +248,10 @@ __global__ void __launch_bounds__(TMAX) k_atencao4_back(const int8_t* __restrict
 // sequences x 128 tokens and 64 heads of 4: forward 25 -> 16 us, backward 36 -> 24 against 8 lanes per query row (24-bit
 // products, operands read from LDS per pair); at 13 x 256 tokens and 32 heads, against one row per thread, forward and
 // backward with both quantizations 303 -> 75 us. A wave per stripe measured 15 and 25 us, and 28 before neighbouring
-// heads shared an XCD; at most 64 registers in the backward (8 waves per SIMD) spilled 24 of them: 35 us.
+// heads shared an XCD; at most 64 registers in the backward (8 waves per SIMD) spilled 24 of them: 35 us. At 16 x 256 tokens
+// and 64 heads 50 and 84 us, the vector unit half busy: 164 registers forward and 114 backward leave 3 and 4 waves per SIMD.
+// One to three sequences of 96 tokens or fewer and 32 heads leave CUs idle either way; there 8 lanes per row had more waves
+// on a head: backward 8.3-10.1 us with them, 8.7-9.9 here, forward 6.0-7.5 and 6.1-7.2.
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 typedef short s2_t __attribute__((ext_vector_type(2)));

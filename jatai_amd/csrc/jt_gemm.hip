@@ -14,9 +14,10 @@
 // The sum leaves [2^23, 2^24] only where |p| > 2^18 at sa = sb = 0; bit 23 of t's bits then says so (one v_or3 per two
 // values, tested once per stage), and the exact sum is added another way. Per output and K-block: fma, fma, half an
 // add3, half an or3 = 3 VALU operations, against 4 in fp64. This per-block VALU work, not the MFMA, bounds the kernel:
-// per wave and stage of two blocks the compiled loop has 111 VALU instructions where the fp64 form had 150. At M = 16384
-// (N x K): 1536 x 512 94 -> 74 us, 512 x 2048 with the R16 add 122 -> 84, 2048 x 512 ReLU^2 131 -> 112 and its backward
-// 131 -> 103; at M = 2048: 512 x 2048 18.2 -> 15.9, 2048 x 512 18.5 -> 14.6 (launches back to back).
+// per wave and stage of two blocks it issues 126 VALU instructions (counted, 96 of them these) where the fp64 form issued
+// 148. At M = 16384 (N x K), with the tile rows the shapes now take: 1536 x 512 98 -> 80 us, 512 x 2048 with the R16 add
+// 103 -> 82, 2048 x 512 ReLU^2 126 -> 108 and its backward 123 -> 104; the rounding alone, 32-row tiles, 2048 x 512: 108 ->
+// 94. At M = 2048: 512 x 2048 17.8 -> 15.9, 2048 x 512 ReLU^2 18.2 -> 15.9 (launches back to back).
 // At BLK = 128 the rounding is a quarter as frequent and runs in fp64, whose code holds fewer registers there:
 //   g = fma(ldexp(double(p), 4 - sa), 2^-sb, 1.5 * 2^52).
 // ldexp and the product by a power of two are exact, and |p * 2^(4 - sa - sb)| < 2^26 (|p| <= 128 * 128 * BLK),
@@ -25,8 +26,8 @@
 // bits). The row term is a 32-bit ldexp operand and the column term one double per column and block: cvt, ldexp, fma
 // and add. (In fp32 there: 14.7 us against 6.5 at 2048 x 768, K = 256 with two K-splits, from spilled stage registers.)
 //
-// Tiling: a workgroup of 4 R x KS waves owns a BM x 128 output tile, BM = 32 R rows (R = 1 or 2 by the grid, gemm_r in
-// jatai.hip; 2 and 4 where jt_gemm_bm selects them), one 128-column block at BLK=128, four at BLK=32. K is walked in stages of
+// Tiling: a workgroup of 4 R x KS waves owns a BM x 128 output tile, BM = 32 R rows (R = 1, 2 or 4 by the shape, gemm_r_auto
+// in jatai.hip, or as jt_gemm_bm says), one 128-column block at BLK=128, four at BLK=32. K is walked in stages of
 // 64 (BLK=32) or 128 (BLK=128) bytes per row: wave group g (4 R waves) takes stages s = g (mod KS) and stages each
 // one through its own double-buffered LDS tile of BM + 128 rows (BM of A, 128 of B) with coalesced loads, issued
 // two stages ahead of the MFMAs; wave w of the group computes the 32 x 32 sub-tile of rows 32 (w / 4) and columns

@@ -21,7 +21,7 @@ BLK = 128
 E_ZERO = -127
 GA = 4
 ATENCAO_LIMITE = False
-# attention through the workspace entry points (jt_atencao_ws): same outputs, faster at head width 64; False runs
+# attention through the workspace entry points (jt_atencao_ws): same outputs, faster at head widths 64, 32 and 16; False runs
 # the reference ABI's jt_atencao
 ATENCAO_WS = True
 AQUI = os.path.dirname(os.path.abspath(__file__))

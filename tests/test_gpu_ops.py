@@ -116,7 +116,7 @@ ATENCAO4 = [i for i, (n, _) in enumerate(CASOS) if n.startswith("atencao")]
 @pytest.mark.parametrize("i", ATENCAO4, ids=[CASOS[i][0] for i in ATENCAO4])
 def test_caso_atencao_duas_linhas(blk, i, linhas):
     """The reference suite's attention cases with the layouts jt_atencao_linhas forces (jatai_cuda.cu:1091): one
-    query row per thread, and two (rows i and T - 1 - i); the default runs 8 lanes per row. The spec's hashes."""
+    query row per thread, and two (rows i and T - 1 - i); the default runs on matrix cores. The spec's hashes."""
     from jatai_amd import ops as O
     lib = O.carrega_lib()
     lib.jt_atencao_linhas(linhas)
@@ -350,7 +350,7 @@ def test_gemm_relu2_back_t(M, N, K):
                                       (512, 512, 4096, 32)])
 def test_gemm_relu2_t(M, N, K, bm):
     """Mode 3 with the transposed copy of its ReLU^2 output (BLK = 32): h and a equal gemm_relu2's and the copy
-    equals transpoe(a), at the automatic tile (128 rows at config 4's shape) and at forced 64- and 32-row tiles."""
+    equals transpoe(a), at the automatic tile (64 rows at M = N = 2048) and at forced 64- and 32-row tiles."""
     blk = 32
     gpu = GPU(blk, vigiar=True)
     s = lambda t: R.substream(96, f"{M} {N} {K} {t}")
